@@ -16,7 +16,9 @@ OUT = os.path.join(PKG, "libducc_amd.so")
 BUILD = os.path.join(HERE, "_build")
 GEN = os.path.join(HERE, "_gen")
 
-SOURCES = ["params.cpp", "runtime.hip", "api.hip", "sort.hip", "spread.hip",
+# the longest compilations first
+SOURCES = ["fft_f32.hip", "fft_f32_half.hip", "fft_f64.hip",
+           "fft_f64_half.hip", "params.cpp", "runtime.hip", "api.hip", "sort.hip", "spread.hip",
            "interp.hip", "fft.hip", "grid.hip", "chooser.hip", "mlp.hip",
            "c2c.hip", "noalloc.hip", "spread_det.hip", "records.hip",
            "sht.hip", "wgridder.hip"]
@@ -30,7 +32,10 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", f"-I{INCLUDE}", "-I" + HERE,
           "-Wno-unused-variable", "-Wno-unused-but-set-variable"]
 DEVICE = [f"--offload-arch={ARCH}", "-munsafe-fp-atomics",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-          "-fno-gpu-flush-denormals-to-zero"]
+          "-fno-gpu-flush-denormals-to-zero",
+          # k_fft's argument struct has more readers than instcombine's
+          # default 300, and would be copied to scratch memory per lane
+          "-mllvm", "-instcombine-max-copied-from-constant-users=65536"]
 
 
 def gen_kernel_db():

@@ -129,6 +129,7 @@ __device__ __forceinline__ void split3(int64_t q, int64_t K, int64_t inner,
 struct BlueArgs {
   int64_t outer, inner, n;  // n: elements of the index space of the launch
   int L, n2, conj_w, small;
+  double scale;  // MODE 0: factor of the input
 };
 
 // MODE 0: a[o,k,i] = k < L ? x[o,k,i] w'[k] : 0        over (outer, n2, inner)
@@ -136,7 +137,7 @@ struct BlueArgs {
 // MODE 2: x[o,m,i] = w'[m] a[o,m,i]                    over (outer, L, inner)
 // w' = w or conj(w) (the transform's sign)
 template <typename T, int MODE>
-__global__ __launch_bounds__(256) void k_bluestein(Cx<T> *x, Cx<T> *a,
+__global__ __launch_bounds__(256) void k_bluestein(Cx<T> *x, const Cx<T> *src, Cx<T> *a,
                                                    const Cx<T> *tab,
                                                    BlueArgs b) {
   for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < b.n;
@@ -157,7 +158,10 @@ __global__ __launch_bounds__(256) void k_bluestein(Cx<T> *x, Cx<T> *a,
     if (MODE == 0) {
       Cx<T> v;
       if (k < b.L) {
-        v = cx_mul<T>(x[ix], w);
+        v = src[ix];
+        v.x *= (T)b.scale;
+        v.y *= (T)b.scale;
+        v = cx_mul<T>(v, w);
       } else {
         v.x = T(0);
         v.y = T(0);
@@ -230,8 +234,10 @@ void chirp_host(int L, std::vector<double> &w) {
   }
 }
 
-void run_lines(void *data, int64_t outer, int L, int64_t inner, bool fp64,
-               int sign, const void *tw, void *scratch, hipStream_t s);
+using Keep = std::vector<std::shared_ptr<Buf>>;
+void run_lines(void *data, const void *src, double scale, int64_t outer,
+               int L, int64_t inner, bool fp64, int sign, const void *tw,
+               void *scratch, hipStream_t s, Keep &keep);
 
 // Bluestein tables for length L (convolution length n2): the chirp w and
 // B = FFT_n2(b~) / n2 with b~[j] = conj(w_j) (j < L), b~[n2-j] = conj(w_j)
@@ -276,7 +282,8 @@ Blue bluestein_tables(int L, int n2, bool fp64, int sign, hipStream_t s) {
   DMX_HIP(hipMemcpy(b64.p, bt.data(), (size_t)n2 * 16, hipMemcpyHostToDevice));
   if (n2 > FFT_MAXEL64) sc.reset((size_t)n2 * 16);
   auto tw64 = twiddles(n2, true);
-  run_lines(b64.p, 1, n2, 1, true, -1, tw64->p, sc.p, s);
+  Keep keep;  // until the synchronization below
+  run_lines(b64.p, nullptr, 1.0, 1, n2, 1, true, -1, tw64->p, sc.p, s, keep);
   auto Bb = std::make_shared<Buf>((size_t)n2 * esz);
   if (fp64) {
     DMX_HIP(hipMemcpyAsync(Bb->p, b64.p, (size_t)n2 * 16,
@@ -303,17 +310,20 @@ Blue bluestein_tables(int L, int n2, bool fp64, int sign, hipStream_t s) {
 // Stockham FFT of every line of the contiguous array (outer, L, inner) along
 // its middle axis, in place (scratch: as large as the array when L is longer
 // than a workgroup's LDS holds).
-void run_lines(void *data, int64_t outer, int L, int64_t inner, bool fp64,
-               int sign, const void *tw, void *scratch, hipStream_t s) {
+void run_lines(void *data, const void *src, double scale, int64_t outer,
+               int L, int64_t inner, bool fp64, int sign, const void *tw,
+               void *scratch, hipStream_t s, Keep &keep) {
   const size_t esz = fp64 ? 16 : 8;
   FftLaunch p{};
   p.L = L;
   p.tw = tw;
   p.sign = sign;
+  p.scale = scale;
   if (inner == 1) {
     // contiguous lines: all of them along the second launch index
     DMX_ASSERT(outer <= 0x7fffffff, "too many FFT lines");
     p.data = data;
+    p.src = src;
     p.st_ax = 1;
     p.nu = 1;
     p.un1 = 1;
@@ -321,6 +331,14 @@ void run_lines(void *data, int64_t outer, int L, int64_t inner, bool fp64,
     p.nv = (int)outer;
     p.vn1 = p.nv;
     p.st_v = L;
+    const int L1 = scratch ? fft_split_long(L, fp64) : 0;
+    if (L1 > 1) {
+      auto t1 = twiddles(L1, fp64), t2 = twiddles(L / L1, fp64);
+      keep.push_back(t1);
+      keep.push_back(t2);
+      if (fft_long_2pass(p, L1, data, fp64, t1->p, t2->p, tw, s, scratch))
+        return;
+    }
     fft_lineset(p, fp64, scratch, s);
     return;
   }
@@ -329,6 +347,7 @@ void run_lines(void *data, int64_t outer, int L, int64_t inner, bool fp64,
   for (int64_t u0 = 0; u0 < outer; u0 += chunk) {
     const int64_t off = u0 * (int64_t)L * inner;
     p.data = (char *)data + off * esz;
+    p.src = src ? (const char *)src + off * esz : nullptr;
     p.st_ax = inner;
     p.nu = (int)std::min<int64_t>(chunk, outer - u0);
     p.un1 = p.nu;
@@ -342,7 +361,7 @@ void run_lines(void *data, int64_t outer, int L, int64_t inner, bool fp64,
 
 // the two-pass column FFT of (outer, L, inner) along its middle axis:
 // pass A data -> scratch, pass B scratch -> data (same layout)
-void run_columns(void *data, int64_t outer, int L, int L1, int64_t inner,
+void run_columns(void *data, const void *src, double scale, int64_t outer, int L, int L1, int64_t inner,
                  bool fp64, int sign, const void *tw1, const void *tw2,
                  const void *tw, void *scratch, hipStream_t s) {
   const size_t esz = fp64 ? 16 : 8;
@@ -354,6 +373,8 @@ void run_columns(void *data, int64_t outer, int L, int L1, int64_t inner,
     p.L = L;
     p.sign = sign;
     p.data = (char *)data + off * esz;
+    p.src = src ? (const char *)src + off * esz : nullptr;
+    p.scale = scale;
     p.st_ax = inner;
     p.nu = (int)std::min<int64_t>(chunk, outer - u0);
     p.un1 = p.nu;
@@ -449,10 +470,11 @@ void copy_nd(const void *src, int src_tc, const int64_t *sst, void *dst,
 }
 
 template <typename T, int MODE>
-void launch_blue(void *x, void *a, const void *tab, const BlueArgs &b,
+void launch_blue(void *x, const void *src, void *a, const void *tab, const BlueArgs &b,
                  hipStream_t s) {
   hipLaunchKernelGGL((k_bluestein<T, MODE>), dim3(grid_for(b.n)), dim3(256), 0,
-                     s, (Cx<T> *)x, (Cx<T> *)a, (const Cx<T> *)tab, b);
+                     s, (Cx<T> *)x, (const Cx<T> *)src, (Cx<T> *)a,
+                     (const Cx<T> *)tab, b);
   DMX_HIP(hipGetLastError());
 }
 
@@ -492,11 +514,21 @@ std::shared_ptr<void> c2c_exec(const void *in, int in_tc, const int64_t *in_st,
     work = job->work.p;
   }
   Timers tm(s);
-  // in place on a contiguous array without scaling: nothing to copy
-  bool in_contig = in == work && in_tc == (fp64 ? DMX_C128 : DMX_C64);
+  // a contiguous input of the same type is read by the first transform
+  // itself, which applies the factor (4096 x 4096 complex64: a copy of
+  // 52 us of 278 us less); `from` and `scale` are what is still to be read
+  // and applied
+  bool in_contig = in_tc == (fp64 ? DMX_C128 : DMX_C64);
   for (int d = 0; d < ndim; ++d)
     if (shape[d] != 1 && in_st[d] != cst[d]) in_contig = false;
-  if (!(in_contig && fct == 1.0)) {
+  bool any = false;  // a transform of length > 1
+  for (int q = 0; q < naxes; ++q) any = any || shape[axes[q]] > 1;
+  const void *from = work;
+  double scale = 1.0;
+  if (in_contig && (any || (in == work && fct == 1.0))) {
+    from = in;
+    scale = fct;
+  } else {
     tm.begin("copy in");
     if (fp64)
       copy_nd<double>(in, in_tc, in_st, work, cst, ndim, shape, fct, s);
@@ -528,14 +560,16 @@ std::shared_ptr<void> c2c_exec(const void *in, int in_tc, const int64_t *in_st,
         auto t1 = twiddles(L1, fp64), t2 = twiddles(L / L1, fp64);
         job->keep.push_back(t1);
         job->keep.push_back(t2);
-        run_columns(work, outer, L, L1, inner, fp64, sign, t1->p, t2->p,
-                    tw->p, job->scratch.p, s);
+        run_columns(work, from, scale, outer, L, L1, inner, fp64, sign, t1->p,
+                    t2->p, tw->p, job->scratch.p, s);
       } else {
         if (L > maxel && !job->scratch.p) job->scratch.reset((size_t)n * esz);
-        run_lines(work, outer, L, inner, fp64, sign, tw->p, job->scratch.p,
-                  s);
+        run_lines(work, from, scale, outer, L, inner, fp64, sign, tw->p,
+                  L > maxel ? job->scratch.p : nullptr, s, job->keep);
       }
       tm.end();
+      from = work;
+      scale = 1.0;
       continue;
     }
     const int n2 = (int)smooth_length(2 * L64 - 1);
@@ -556,17 +590,22 @@ std::shared_ptr<void> c2c_exec(const void *in, int in_tc, const int64_t *in_st,
     b.conj_w = sign > 0 ? 1 : 0;
     b.n = nb;
     b.small = nb < (1ll << 32) ? 1 : 0;
+    b.scale = scale;
     void *A = job->blue.p;
     tm.begin("Bluestein axis " + std::to_string(ax));
-    if (fp64) launch_blue<double, 0>(work, A, bt.w->p, b, s);
-    else launch_blue<float, 0>(work, A, bt.w->p, b, s);
-    run_lines(A, outer, n2, inner, fp64, -1, tw2->p, job->blue_scratch.p, s);
-    if (fp64) launch_blue<double, 1>(work, A, bt.B->p, b, s);
-    else launch_blue<float, 1>(work, A, bt.B->p, b, s);
-    run_lines(A, outer, n2, inner, fp64, 1, tw2->p, job->blue_scratch.p, s);
+    if (fp64) launch_blue<double, 0>(work, from, A, bt.w->p, b, s);
+    else launch_blue<float, 0>(work, from, A, bt.w->p, b, s);
+    run_lines(A, nullptr, 1.0, outer, n2, inner, fp64, -1, tw2->p,
+              n2 > maxel ? job->blue_scratch.p : nullptr, s, job->keep);
+    if (fp64) launch_blue<double, 1>(work, from, A, bt.B->p, b, s);
+    else launch_blue<float, 1>(work, from, A, bt.B->p, b, s);
+    run_lines(A, nullptr, 1.0, outer, n2, inner, fp64, 1, tw2->p,
+              n2 > maxel ? job->blue_scratch.p : nullptr, s, job->keep);
     b.n = outer * (int64_t)L * inner;
-    if (fp64) launch_blue<double, 2>(work, A, bt.w->p, b, s);
-    else launch_blue<float, 2>(work, A, bt.w->p, b, s);
+    if (fp64) launch_blue<double, 2>(work, from, A, bt.w->p, b, s);
+    else launch_blue<float, 2>(work, from, A, bt.w->p, b, s);
+    from = work;
+    scale = 1.0;
     tm.end();
   }
   if (!out_contig) {

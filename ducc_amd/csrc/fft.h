@@ -10,9 +10,16 @@ namespace dmx {
 #define FFT_THREADS 256
 #define FFT_MAXEL32 8192  // 64 KiB of complex float per workgroup
 #define FFT_MAXEL64 4096  // 64 KiB of complex double per workgroup
-// butterflies per thread and pass for workgroups of at most MAXEL elements
-#define FFT_KM_EL(MAXEL, R) (((MAXEL) + (R)*FFT_THREADS - 1) / ((R)*FFT_THREADS))
-#define FFT_KM(T, R) FFT_KM_EL(sizeof(T) == 8 ? FFT_MAXEL64 : FFT_MAXEL32, R)
+#define FFT_MAXPASS 24
+#define FFT_MIN_GROUPS 512  // workgroups that small line sets aim at
+// butterflies per thread and pass for workgroups of at most MAXEL elements;
+// of the wide composite radices only as many as MAXEL fills (the host uses
+// them for workgroups that this covers)
+constexpr int fft_km(int maxel, int R) {
+  const int d = R * FFT_THREADS;
+  if (R == 12 || R == 14 || R == 15) return maxel >= d ? maxel / d : 1;
+  return (maxel + d - 1) / d;
+}
 
 // Constants of one Stockham pass, computed on the host: radix, butterflies
 // per line (L/R), sub-transform length before the pass (Ns), twiddle stride
@@ -21,18 +28,17 @@ struct FftPass {
   int radix, nbf, ns, twstep;
   float inv_nbf, inv_ns;
 };
-// fills pass[0..npass) for a line of length L; returns npass
-int fft_plan_passes(int L, FftPass *pass, int maxpass);
-
 // Lines along one axis of a row-major array.  Line (u, v) starts at
 // U(u)*st_u + V(v)*st_v, element k at + k*st_ax, where the virtual indices
 // map to actual ones through at most two ranges:
 // U(u) = u < un1 ? ua1 + u : ua2 + (u - un1)   (same for V).
 struct FftLaunch {
-  void *data;
+  void *data;       // result (and input, in place)
+  const void *src;  // input at the same positions (null: data)
+  double scale;     // the input's factor (0: one)
   const void *tw;  // exp(-2 pi i m / L), m < L, compute type
-  int L, LP, Bl, npass, sign;
-  FftPass pass[24];
+  int L, npass, sign;
+  FftPass pass[FFT_MAXPASS];
   int64_t st_ax, st_u, st_v;
   int nu, nv;
   int un1, ua1, ua2, vn1, va1, va2;
@@ -57,23 +63,31 @@ struct FftCrop {
   int fft_order, u_f64;
 };
 
-// One half of the two-pass FFT along a strided axis (see k_fft_cols).
-struct FftCols {
+// One launch of k_fft: nv lines b (virtual -> actual through a range, as
+// above) for every u (blockIdx.y) and outer index (blockIdx.z).  Element e
+// of a line is read at src + z*st_o + u*in_u + b*in_b + e*in_e and has the
+// natural index u*nin_u + b*nin_b + e*nin_e (zero in the k range); result k goes to dst
+// with the out_ / nout_ numbers (not stored in the s range), times w_L^(k * u) (twiddle 1) or
+// w_L^(k * b) (twiddle 2), or through the crop.
+struct FftArgs {
   const void *src;
   void *dst;
-  const void *tw_sub;   // twiddles of length Lsub
-  const void *tw_full;  // twiddles of length L (inter-pass factors)
-  int L, Lsub, npass, sign, twiddle, Bl;
-  FftPass pass[24];
-  int64_t ia, ib, oa, ob;  // row maps of input / output (in rows)
-  int64_t rs;              // row stride (elements)
-  int ncol, vn1, va1, va2; // columns (virtual -> actual, stride 1)
-  int nlines;
-  int nouter, on1, oa1, oa2;
-  int64_t st_o;
-  int sprune, sn1, sa2;  // output rows sn1 <= row < sa2 are not stored
-  int kprune, kn1, ka2;  // input rows kn1 <= row < ka2 are read as zero
-  int crop;              // store through `cr` instead of dst (pass B)
+  const void *tw;       // twiddles of length Ls
+  const void *tw_full;  // twiddles of length L (twiddle)
+  double scale;         // factor of the input
+  int Ls, LP, Bl, npass;
+  FftPass pass[FFT_MAXPASS];
+  int nv, vn1, va1, va2;
+  int un1, ua1, ua2;
+  int on1, oa1, oa2;
+  int64_t in_b, in_e, in_u, out_b, out_k, out_u, st_o;
+  int nin_b, nin_e, nin_u, nout_b, nout_k, nout_u;
+  int kn1, kspan, sn1, sspan;  // pruned: [kn1, kn1 + kspan), ...
+  int twiddle, tw_lds;
+  // butterflies dealt with the line index running fastest (lines side by
+  // side in memory) in the first, middle and last passes
+  int bf_in, bf_mid, bf_out;
+  int crop;
   FftCrop cr;
 };
 
@@ -91,6 +105,15 @@ bool fft_columns_2pass(const FftLaunch &p, int L1, void *dst, bool fp64,
                        void *a_dst = nullptr, const FftCrop *crop = nullptr);
 // a divisor of L near sqrt(L) with both factors <= 128 (0: none)
 int fft_split(int L);
+
+// The same over contiguous lines (st_ax == 1) too long for LDS, or too few
+// to fill the chip one workgroup a line; natural order in and out, pass A in
+// place (or into a_dst), dst must not be pass A's output.
+bool fft_long_2pass(const FftLaunch &p, int L1, void *dst, bool fp64,
+                    const void *tw_L1, const void *tw_L2, const void *tw_L,
+                    hipStream_t s, void *a_dst = nullptr);
+// the divisor of L that fft_long_2pass takes (0: none)
+int fft_split_long(int L, bool fp64);
 
 void fft_twiddles(int L, bool fp64, std::vector<unsigned char> &out);
 // the same table computed on the device into dst (L complex values of the

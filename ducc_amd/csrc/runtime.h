@@ -268,8 +268,9 @@ class Plan {
   std::string tag_ = "plan";  // "index", "nu2u" or "u2nu": phase prefix
   void prepare_grid_side();
   // how the FFT along real axis d runs: in LDS, as the two-pass 2-D column
-  // FFT, or as global passes (lines longer than LDS)
-  enum class FftRoute { none, lds, columns, global };
+  // FFT, as two passes over long rows, or as global passes (lines longer
+  // than LDS)
+  enum class FftRoute { none, lds, columns, rows, global };
   FftRoute fft_route(int d) const;
   GridCopyArgs copy_args(const void *uni, bool uni_f64,
                          const int64_t *ust) const;

@@ -569,9 +569,21 @@ std::shared_ptr<Setup> Plan::arena_setup(const Params &p, hipStream_t s) {
 }
 
 namespace {
+// Lines along the last axis that take two passes (fft_long_2pass): those
+// beyond LDS, and a single line of 1024 elements or more, whose passes one
+// workgroup would run alone (185220 points: eight passes through memory,
+// 33 us, against two of 6 us)
+// (in the static arena of the allocation-free entry points, whose size is
+// fixed, lines take the routes that need no second array)
+bool long_rows(const Params &p, int d, bool arena) {
+  const int L = (int)p.nover[d], maxel = p.fp64 ? FFT_MAXEL64 : FFT_MAXEL32;
+  return !arena && d == p.ndim - 1 && (L > maxel || (p.ndim == 1 && L >= 1024)) &&
+         fft_split_long(L, p.fp64) > 1;
+}
 // the distinct FFT lengths whose twiddles a transform uses: each axis's
 // length, plus the two factors of the two-pass column FFT
-void fft_lengths(const Params &p, bool has_scratch, std::vector<int> &Ls) {
+void fft_lengths(const Params &p, bool has_scratch, bool arena,
+                 std::vector<int> &Ls) {
   const int maxel = p.fp64 ? FFT_MAXEL64 : FFT_MAXEL32;
   auto add = [&](int L) {
     if (std::find(Ls.begin(), Ls.end(), L) == Ls.end()) Ls.push_back(L);
@@ -584,13 +596,19 @@ void fft_lengths(const Params &p, bool has_scratch, std::vector<int> &Ls) {
       add(fft_split(L));
       add(L / fft_split(L));
     }
+    if (long_rows(p, d, arena) && has_scratch) {
+      add(fft_split_long(L, p.fp64));
+      add(L / fft_split_long(L, p.fp64));
+    }
     add(L);
   }
 }
-bool needs_scratch_grid(const Params &p) {
+bool needs_scratch_grid(const Params &p, bool arena) {
   bool need = p.ndim == 2;
   for (int d = 0; d < p.ndim; ++d)
-    if ((int)p.nover[d] > (p.fp64 ? FFT_MAXEL64 : FFT_MAXEL32)) need = true;
+    if ((int)p.nover[d] > (p.fp64 ? FFT_MAXEL64 : FFT_MAXEL32) ||
+        long_rows(p, d, arena))
+      need = true;
   return need;
 }
 }  // namespace
@@ -618,11 +636,11 @@ size_t Plan::scratch_bytes(const Params &p, size_t M) {
   // grid side (prepare_grid_side)
   size_t n = 1;
   for (int d = 0; d < p.ndim; ++d) n *= p.nover[d];
-  const bool scr = needs_scratch_grid(p);
+  const bool scr = needs_scratch_grid(p, true);
   b += round256(n * esz) * (scr ? 2 : 1);
   // twiddles (twiddle_for)
   std::vector<int> Ls;
-  fft_lengths(p, scr, Ls);
+  fft_lengths(p, scr, true, Ls);
   for (int L : Ls) b += round256((size_t)L * esz);
   return b;
 }
@@ -822,7 +840,7 @@ void Plan::prepare_grid_side() {
   // the second buffer serves lines longer than LDS and the out-of-place
   // half of the two-pass column FFT (2-D)
   scratch_.stream = s_;
-  if (needs_scratch_grid(p_) && scratch_.bytes != bytes) scratch_.reset(bytes);
+  if (needs_scratch_grid(p_, current_arena() != nullptr) && scratch_.bytes != bytes) scratch_.reset(bytes);
   cur_ = grid_.p;
 }
 
@@ -855,6 +873,7 @@ Plan::FftRoute Plan::fft_route(int d) const {
   if (p_.ndim == 2 && d == 0 && maxel / L < 16 && fft_split(L) > 0 &&
       scratch_.p)
     return FftRoute::columns;
+  if (long_rows(p_, d, current_arena() != nullptr) && scratch_.p) return FftRoute::rows;
   return L <= maxel ? FftRoute::lds : FftRoute::global;
 }
 
@@ -903,7 +922,6 @@ bool Plan::run_fft(bool forward, bool type1, const GridCopyArgs *crop) {
   std::vector<int> order;
   if (type1) for (int a = 2; a >= f; --a) order.push_back(a);
   else for (int a = f; a <= 2; ++a) order.push_back(a);
-  const int maxel = p_.fp64 ? FFT_MAXEL64 : FFT_MAXEL32;
   for (int a : order) {
     int pax = a == 0 ? 1 : 0, qax = a == 2 ? 1 : 2;
     FftLaunch L{};
@@ -936,8 +954,10 @@ bool Plan::run_fft(bool forward, bool type1, const GridCopyArgs *crop) {
       // two coalesced passes (64 columns per workgroup), the second writing
       // natural order into the other buffer
       void *other = cur_ == grid_.p ? scratch_.p : grid_.p;
-      // rows longer than LDS cannot skip the unwritten columns: clear them
-      if (!type1 && E[2] > maxel) launch_zero(other, grid_.bytes, s_);
+      // rows done by global passes cannot skip the unwritten columns: clear
+      // them
+      if (!type1 && fft_route(nd - 1) == FftRoute::global)
+        launch_zero(other, grid_.bytes, s_);
       const int L1 = fft_split(L.L);
       // type 1, 2-D: the column pass is the last one; it writes the
       // retained modes to the uniform array with their correction factors
@@ -962,6 +982,16 @@ bool Plan::run_fft(bool forward, bool type1, const GridCopyArgs *crop) {
       cur_ = other;
       cropped = cropped || fuse;
       continue;
+    }
+    if (route == FftRoute::rows) {
+      void *other = cur_ == grid_.p ? scratch_.p : grid_.p;
+      const int L1 = fft_split_long(L.L, p_.fp64);
+      if (fft_long_2pass(L, L1, other, p_.fp64, twiddle_for(L1),
+                         twiddle_for(L.L / L1), twiddle_for(L.L), s_)) {
+        cur_ = other;
+        continue;
+      }
+      DMX_ASSERT(false, "FFT line set too large");
     }
     L.tw = twiddle_for(L.L);
     fft_lineset(L, p_.fp64, cur_ == grid_.p ? scratch_.p : grid_.p, s_);

@@ -1,0 +1,77 @@
+"""GPU: the FFT passes at their edges - every radix alone and combined, line
+counts that leave a workgroup partly filled, lines that take two passes over
+L1 x L2, out-of-place input with a factor - against a 64-bit FFT."""
+import numpy as np
+import pytest
+import torch
+
+from ducc_amd import fft, nufft
+
+pytestmark = pytest.mark.gpu
+
+# one length per radix, composite pairs, the longest lines in LDS, and lines
+# beyond it (two passes; 16381 is prime: Bluestein over a long line)
+LENGTHS = [2, 3, 5, 6, 7, 9, 10, 11, 12, 14, 15, 16, 84, 110, 210, 432, 462,
+           1078, 1210, 1440, 3388, 3750, 3840, 4096, 7168, 8192, 8232, 11025,
+           16381, 185220]
+
+
+def tol(dtype, n):
+    """rounding of log2(n) butterfly levels and their twiddles, in rms"""
+    eps = 1.2e-7 if dtype == torch.complex64 else 2.3e-16
+    return 4 * eps * np.log2(max(n, 2))
+
+
+@pytest.mark.parametrize("dtype", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("n", LENGTHS)
+def test_lines(n, dtype):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    for shape, ax in (((1, n), 1), ((7, n), 1), ((n, 1), 0), ((n, 37), 0),
+                      ((2, n, 5), 1)):
+        if n > 20000 and shape[0] * shape[-1] > 7 * n:
+            continue
+        a = torch.randn(shape, dtype=dtype, device="cuda", generator=g)
+        keep = a.clone()
+        for fwd in (True, False):
+            r = fft.c2c(a, axes=[ax], forward=fwd, inorm=0 if fwd else 2)
+            f = torch.fft.fft if fwd else torch.fft.ifft
+            e = f(a.to(torch.complex128), dim=ax)
+            err = ((r - e).norm() / e.norm()).item()
+            # Bluestein: three transforms of twice the length
+            assert err < tol(dtype, n) * (4 if n == 16381 else 1), (shape, err)
+            assert torch.equal(a, keep)
+
+
+@pytest.mark.parametrize("n,eps,dtype,coord", [
+    (700, 1e-5, torch.complex64, torch.float32),
+    (5000, 1e-9, torch.complex128, torch.float64),
+    (9001, 1e-5, torch.complex64, torch.float64),
+    (100003, 1e-4, torch.complex64, torch.float64),
+    (60000, 1e-9, torch.complex128, torch.float64)])
+def test_long_rows_nufft(n, eps, dtype, coord):
+    """1-D transforms whose grid is one long line, both types and orders"""
+    rng = np.random.default_rng(n)
+    M = 300
+    x = rng.uniform(-np.pi, np.pi, M)
+    x = x.astype(np.float32 if coord == torch.float32 else np.float64)
+    k = np.arange(n) - n // 2
+    E = np.exp(1j * np.outer(x.astype(np.float64), k))
+    p = rng.standard_normal(M) + 1j * rng.standard_normal(M)
+    c = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    xt = torch.from_numpy(x).cuda()[:, None]
+    pt = torch.from_numpy(p).cuda().to(dtype)
+    ct = torch.from_numpy(c).cuda().to(dtype)
+    # float32 coordinates are folded in double: no error beyond eps
+    lim = 4 * eps + (2e-6 if dtype == torch.complex64 else 1e-13)
+    for fo in (False, True):
+        sh = (lambda a: np.fft.ifftshift(a)) if fo else (lambda a: a)
+        out = torch.empty(n, dtype=dtype, device="cuda")
+        nufft.nu2u(points=pt, coord=xt, forward=True, epsilon=eps, out=out,
+                   fft_order=fo)
+        e = sh(E.conj().T @ p)
+        assert np.linalg.norm(out.cpu().numpy() - e) <= lim * np.linalg.norm(e)
+        g = torch.from_numpy(sh(ct.cpu().numpy()).copy()).cuda()
+        v = nufft.u2nu(grid=g, coord=xt, forward=False, epsilon=eps,
+                       fft_order=fo)
+        e = E @ c
+        assert np.linalg.norm(v.cpu().numpy() - e) <= lim * np.linalg.norm(e)
