@@ -254,6 +254,14 @@ void launch_tile_subs(size_t ntiles, uint32_t *counts, uint32_t *tstart,
                       const uint32_t *tend, uint32_t *nsub,
                       uint32_t *sub_start, Sub *subs, uint32_t *nsub_total,
                       void *scanwork, hipStream_t s);
+// the whole index build (order, tile tables, subproblems) where one counting
+// pass over whole tile keys does it: few tiles, and a table that fits the
+// workspace of the 8-bit passes (`work`).  false: nothing was launched.
+bool launch_index(const Geo &g, const void *coords, size_t M, int keybits,
+                  size_t ntiles, uint32_t *idx, uint32_t *keys, void *work,
+                  uint32_t *counts, uint32_t *tstart, uint32_t *nsub,
+                  uint32_t *sub_start, Sub *subs, uint32_t *nsub_total,
+                  hipStream_t s);
 void launch_gather_coords(const void *coords, int coord_f32, int ndim,
                           const uint32_t *idx, size_t M, void *out,
                           hipStream_t s);

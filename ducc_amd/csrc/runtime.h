@@ -308,11 +308,13 @@ class Plan {
   bool rec_ = false, rec_type1_ = false;
   RecBufs recs_{};
   Buf rec_buf_, rec_tmp_;
-  // the tile tables and subproblem list from the sort's tile ranges
+  // room for the subproblem list; the tile tables and the list from the
+  // 8-bit passes' tile ranges
+  void alloc_subs(uint32_t *tables);
   void finish_index(uint32_t *tables);
   Buf tmp_keys_, tmp_tiles_, tmp_work_;
   Buf grid_, scratch_, slab_;
-  const uint32_t *tile_nsub_ = nullptr, *tile_sub0_ = nullptr;
+  uint32_t *tile_nsub_ = nullptr, *tile_sub0_ = nullptr;
   void *cur_ = nullptr;  // buffer holding the grid after the FFT passes
   const void *twiddle_for(int L);
 };

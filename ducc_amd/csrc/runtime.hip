@@ -705,14 +705,22 @@ void Plan::build_index(const void *coords, bool coord_f32, size_t M,
            *tend = tstart + ntiles_;
   {
     Phase ph(this, "building index");
-    launch_zero(tstart, ntiles_ * 8, s_);  // tstart and tend, adjacent
-    launch_fold_keys(g_, coords, M, tmp_keys_.as<uint32_t>(),
-                     radix_sort_hist0(tmp_work_.p, M), s_);
     idx_.stream = s_;
     idx_.reset(M * 4);
-    radix_sort_pairs(tmp_keys_.as<uint32_t>(), M, keybits, idx_.as<uint32_t>(),
-                     nullptr, tmp_work_.p, ws, s_, true, tstart, tend);
-    finish_index(counts);
+    alloc_subs(counts);
+    // few tiles: one counting pass over whole keys; else 8-bit passes
+    if (!launch_index(g_, coords, M, keybits, ntiles_, idx_.as<uint32_t>(),
+                      tmp_keys_.as<uint32_t>(), tmp_work_.p, counts, tstart,
+                      tile_nsub_, tile_sub0_, subs_.as<Sub>(),
+                      nsub_total_.as<uint32_t>(), s_)) {
+      launch_zero(tstart, ntiles_ * 8, s_);  // tstart and tend, adjacent
+      launch_fold_keys(g_, coords, M, tmp_keys_.as<uint32_t>(),
+                       radix_sort_hist0(tmp_work_.p, M), s_);
+      radix_sort_pairs(tmp_keys_.as<uint32_t>(), M, keybits,
+                       idx_.as<uint32_t>(), nullptr, tmp_work_.p, ws, s_,
+                       true, tstart, tend);
+      finish_index(counts);
+    }
   }
   if (keep_sorted_coords) {
     // a random gather of 1e7 points costs about as much as the gathers it
@@ -728,19 +736,22 @@ void Plan::build_index(const void *coords, bool coord_f32, size_t M,
   }
 }
 
-void Plan::finish_index(uint32_t *counts) {
-  uint32_t *tstart = counts + ntiles_, *tend = tstart + ntiles_,
-           *nsub = tend + ntiles_, *sstart = nsub + ntiles_;
+void Plan::alloc_subs(uint32_t *counts) {
+  tile_nsub_ = counts + 3 * ntiles_;
+  tile_sub0_ = counts + 4 * ntiles_;
   nsub_max_ = std::min(ntiles_, M_) + (M_ + MAXSUB - 1) / MAXSUB;
   subs_.stream = s_;
   subs_.reset(nsub_max_ * sizeof(Sub));
   nsub_total_.stream = s_;
   nsub_total_.reset(4);
-  launch_tile_subs(ntiles_, counts, tstart, tend, nsub, sstart,
+}
+
+// after the 8-bit passes: the tile table and the subproblems
+void Plan::finish_index(uint32_t *counts) {
+  uint32_t *tstart = counts + ntiles_, *tend = tstart + ntiles_;
+  launch_tile_subs(ntiles_, counts, tstart, tend, tile_nsub_, tile_sub0_,
                    subs_.as<Sub>(), nsub_total_.as<uint32_t>(), tmp_work_.p,
                    s_);
-  tile_nsub_ = nsub;
-  tile_sub0_ = sstart;
 }
 
 bool Plan::build_records(const void *coords, bool coord_f32, size_t M,
@@ -779,6 +790,7 @@ bool Plan::build_records(const void *coords, bool coord_f32, size_t M,
            *tend = tstart + ntiles_;
   {
     Phase ph(this, "building index");
+    alloc_subs(counts);
     launch_zero(tstart, ntiles_ * 8, s_);  // tstart and tend, adjacent
     rec_sort(g_, offbits, keybits, p_.fp64, type1, coords, values,
              values_f64 ? 1 : 0, M, recs_, tmp, tmp_work_.p, ws, tstart, tend,

@@ -285,6 +285,10 @@ __global__ __launch_bounds__(ST) void k_tile_subs_one(
     uint32_t ev[TS_ITEMS], sv[TS_ITEMS];
 #pragma unroll
     for (int k = 0; k < TS_ITEMS; ++k) {
+      if (k * ST >= nc) {
+        ev[k] = sv[k] = 0;
+        continue;
+      }
       const size_t t = c + (size_t)min(k * ST + tid, nc - 1);
       ev[k] = tend[t];
       sv[k] = tstart[t];
@@ -362,6 +366,339 @@ __global__ __launch_bounds__(ST) void k_tile_subs_one(
     carry += tot;
   }
   if (tid == 0) *nsub_total = carry;
+}
+
+// ------------------------------------------------- one workgroup, one launch
+// Index build of at most SMALL_M points in at most SMALL_TILES tiles: fold,
+// stable LSD sort, tile table and subproblems by one workgroup of 1024
+// threads in LDS.  Such a request is a chain of launch latencies: six
+// launches of 2-9 us each took 27 us for 2000 points, this one 9 us.
+constexpr int SMALL_T = 1024, SMALL_I = 4, SMALL_M = SMALL_T * SMALL_I,
+              SMALL_TILES = 4096, SMALL_W = SMALL_T / 64;
+
+// exclusive prefix over 1024 threads
+__device__ __forceinline__ uint32_t scan1024(uint32_t v, uint32_t *sh,
+                                             uint32_t &total) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  uint32_t x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, (unsigned)o);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) sh[w] = x;
+  __syncthreads();
+  uint32_t before = 0, tot = 0;
+#pragma unroll
+  for (int i = 0; i < SMALL_W; ++i) {
+    const uint32_t s = sh[i];
+    before += i < w ? s : 0u;
+    tot += s;
+  }
+  total = tot;
+  __syncthreads();
+  return before + x - v;
+}
+
+// lanes of the wave with the same value of the low `bits` bits
+__device__ __forceinline__ unsigned long long peers_of(uint32_t d, bool valid,
+                                                       int bits) {
+  unsigned long long peers = __ballot(valid);
+  for (int b = 0; b < bits; ++b) {
+    const bool bit = (d >> b) & 1;
+    const unsigned long long bal = __ballot(bit);
+    peers &= bit ? bal : ~bal;
+  }
+  return peers;
+}
+
+template <int NDIM>
+__device__ __forceinline__ uint32_t tile_key(const Geo &g, const double *x) {
+  uint32_t key = 0;
+#pragma unroll
+  for (int d = 0; d < NDIM; ++d) {
+    double fr;
+    const int c0 = fold_axis(g, d, x[d], fr);
+    const uint32_t t = (uint32_t)((c0 + g.nsafe) >> g.log2tile);
+    key = d == 0 ? t : key * (uint32_t)g.ntiles[d] + t;
+  }
+  return key;
+}
+
+template <int NDIM>
+__global__ __launch_bounds__(SMALL_T) void k_index_small(
+    Geo g, const void *coords, int M, int keybits, int ntiles,
+    uint32_t *idx_out, uint32_t *counts, uint32_t *tstart, uint32_t *nsub,
+    uint32_t *sstart, Sub *subs, uint32_t *nsub_total) {
+  __shared__ uint32_t skey[SMALL_M];
+  __shared__ uint16_t sidx[SMALL_M];
+  __shared__ union {
+    uint32_t cnt[SMALL_W][256];  // digits of a wave's items (sort)
+    struct {
+      uint32_t st[SMALL_TILES], en[SMALL_TILES];  // tile ranges (after it)
+    } t;
+  } u;
+  __shared__ uint32_t sh[SMALL_W];
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const unsigned lane = lane_id();
+  const unsigned long long below_mask =
+      lane ? (~0ull >> (64 - lane)) : 0ull;
+  // item r of lane l of wave w is number w*256 + r*64 + l
+  const int q0 = wave * (64 * SMALL_I) + (int)lane;
+  uint32_t key[SMALL_I], id[SMALL_I];
+  bool valid[SMALL_I];
+  {
+    double x[SMALL_I][NDIM];
+#pragma unroll
+    for (int r = 0; r < SMALL_I; ++r) {
+      id[r] = (uint32_t)(q0 + r * 64);
+      valid[r] = (int)id[r] < M;
+      if (valid[r]) load_point(g, coords, (size_t)id[r], NDIM, x[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < SMALL_I; ++r)
+      key[r] = valid[r] ? tile_key<NDIM>(g, x[r]) : 0u;
+  }
+  for (int shift = 0; shift < keybits; shift += 8) {
+    const int bits = min(8, keybits - shift);
+    for (int c = tid; c < SMALL_W * 256; c += SMALL_T) u.cnt[0][c] = 0;
+    __syncthreads();
+    uint32_t rank[SMALL_I], dig[SMALL_I];
+#pragma unroll
+    for (int r = 0; r < SMALL_I; ++r) {
+      dig[r] = (key[r] >> shift) & 0xFFu;
+      const unsigned long long peers = peers_of(dig[r], valid[r], bits);
+      const unsigned long long below = peers & below_mask;
+      const uint32_t old = u.cnt[wave][dig[r]];
+      __builtin_amdgcn_wave_barrier();
+      if (valid[r] && below == 0)
+        u.cnt[wave][dig[r]] = old + (uint32_t)__popcll(peers);
+      __builtin_amdgcn_wave_barrier();
+      rank[r] = old + (uint32_t)__popcll(below);
+    }
+    __syncthreads();
+    // digit tid: its items in the waves before, its start in the block
+    uint32_t run = 0, tot;
+    if (tid < 256) {
+#pragma unroll
+      for (int w = 0; w < SMALL_W; ++w) {
+        const uint32_t c = u.cnt[w][tid];
+        u.cnt[w][tid] = run;
+        run += c;
+      }
+    }
+    const uint32_t start = scan1024(run, sh, tot);
+    if (tid < 256) {
+#pragma unroll
+      for (int w = 0; w < SMALL_W; ++w) u.cnt[w][tid] += start;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < SMALL_I; ++r) {
+      if (!valid[r]) continue;
+      const uint32_t p = u.cnt[wave][dig[r]] + rank[r];
+      skey[p] = key[r];
+      sidx[p] = (uint16_t)id[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < SMALL_I; ++r) {
+      const int q = q0 + r * 64;
+      if (!valid[r]) continue;  // positions and items end at M alike
+      key[r] = skey[q];
+      id[r] = sidx[q];
+    }
+  }
+  for (int c = tid; c < SMALL_TILES; c += SMALL_T) u.t.st[c] = u.t.en[c] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < SMALL_I; ++r) {
+    const int q = q0 + r * 64;
+    if (!valid[r]) continue;
+    idx_out[q] = id[r];
+    if (q == 0 || skey[q - 1] != key[r]) u.t.st[key[r]] = (uint32_t)q;
+    if (q == M - 1 || skey[q + 1] != key[r]) u.t.en[key[r]] = (uint32_t)q + 1;
+  }
+  __syncthreads();
+  // four consecutive tiles per thread
+  constexpr int TI = SMALL_TILES / SMALL_T;
+  uint32_t ns[TI], sum = 0, tot;
+#pragma unroll
+  for (int k = 0; k < TI; ++k) {
+    const int t = tid * TI + k;
+    ns[k] = (u.t.en[t] - u.t.st[t] + MAXSUB - 1) / MAXSUB;
+    sum += ns[k];
+  }
+  uint32_t ex = scan1024(sum, sh, tot);
+#pragma unroll
+  for (int k = 0; k < TI; ++k) {
+    const int t = tid * TI + k;
+    if (t >= ntiles) break;
+    const uint32_t a = u.t.st[t], e = u.t.en[t];
+    tstart[t] = a;
+    counts[t] = e - a;
+    nsub[t] = ns[k];
+    sstart[t] = ex;
+    for (uint32_t q = 0; q < ns[k]; ++q) {
+      Sub sb;
+      sb.tile = (uint32_t)t;
+      sb.start = a + q * MAXSUB;
+      sb.end = min(e, sb.start + (uint32_t)MAXSUB);
+      sb.rank = q;
+      subs[ex + q] = sb;
+    }
+    ex += ns[k];
+  }
+  if (tid == 0) *nsub_total = tot;
+}
+
+// ------------------------------------------------ one pass, whole keys
+// Index build in one stable counting pass whose digit is the whole tile key
+// (at most WIDE_TILES tiles): fold + histogram, chunk scans, the scan of the
+// chunk sums with the tile table (a tile's start is its first table entry)
+// and subproblems, scatter: four launches and one trip of the points where
+// the 8-bit passes take ten launches and two.  1e6 points in 364 tiles:
+// 62 -> 39 us; 1e5 points in 289 tiles: 60 -> 21 us; 2e6 points in 1600
+// tiles: 87 -> 69 us.
+constexpr int WIDE_TILES = 4096;
+
+template <int NDIM, int ITEMS>
+__global__ __launch_bounds__(RT) void k_fold_wide(Geo g, const void *coords,
+                                                  size_t M, uint32_t *keys,
+                                                  uint32_t *hist, int nbins,
+                                                  int nblocks) {
+  extern __shared__ uint32_t h[];
+  const int tid = threadIdx.x;
+  for (int c = tid; c < nbins; c += RT) h[c] = 0;
+  __syncthreads();
+  const size_t base = (size_t)blockIdx.x * (RT * ITEMS) + tid;
+  double x[ITEMS][NDIM];
+#pragma unroll
+  for (int q = 0; q < ITEMS; ++q) {
+    const size_t j = base + (size_t)q * RT;
+    if (j < M) load_point(g, coords, j, NDIM, x[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < ITEMS; ++q) {
+    const size_t j = base + (size_t)q * RT;
+    if (j >= M) continue;
+    const uint32_t key = tile_key<NDIM>(g, x[q]);
+    keys[j] = key;
+    atomicAdd(&h[key], 1u);
+  }
+  __syncthreads();
+  for (int c = tid; c < nbins; c += RT)
+    hist[(size_t)c * nblocks + blockIdx.x] = h[c];
+}
+
+// The scan of the table's chunk sums, the tile table and the subproblems, by
+// one workgroup: tile t starts at the table's entry t * nblocks.
+constexpr int WIDE_CHUNKS = 4096;
+__global__ __launch_bounds__(1024) void k_tiles_wide(
+    const uint32_t *offs, uint32_t *bsum, int nch, size_t M, int ntiles,
+    int nblocks, uint32_t *counts, uint32_t *tstart, uint32_t *nsub,
+    uint32_t *sstart, Sub *subs, uint32_t *nsub_total) {
+  __shared__ uint32_t sb_[WIDE_CHUNKS], sh[SMALL_W];
+  const int tid = threadIdx.x;
+  uint32_t carry = 0, tot;
+  for (int c = 0; c < nch; c += 1024) {
+    const int i = c + tid;
+    const uint32_t v = i < nch ? bsum[i] : 0u;
+    const uint32_t x = scan1024(v, sh, tot) + carry;
+    if (i < nch) sb_[i] = bsum[i] = x;
+    carry += tot;
+  }
+  __syncthreads();
+  carry = 0;
+  for (int c = 0; c < ntiles; c += 1024) {
+    const int t = c + tid;
+    uint32_t a = 0, e = 0;
+    if (t < ntiles) {
+      const size_t o0 = (size_t)t * nblocks, o1 = o0 + nblocks;
+      a = offs[o0] + sb_[o0 / STILE];
+      e = t + 1 < ntiles ? offs[o1] + sb_[o1 / STILE] : (uint32_t)M;
+      if (a == e) a = e = 0;  // an empty tile
+    }
+    const uint32_t ns = (e - a + MAXSUB - 1) / MAXSUB;
+    const uint32_t ex = scan1024(ns, sh, tot) + carry;
+    carry += tot;
+    if (t < ntiles) {
+      tstart[t] = a;
+      counts[t] = e - a;
+      nsub[t] = ns;
+      sstart[t] = ex;
+      for (uint32_t q = 0; q < ns; ++q) {
+        Sub sb;
+        sb.tile = (uint32_t)t;
+        sb.start = a + q * MAXSUB;
+        sb.end = min(e, sb.start + (uint32_t)MAXSUB);
+        sb.rank = q;
+        subs[ex + q] = sb;
+      }
+    }
+  }
+  if (tid == 0) *nsub_total = carry;
+}
+
+// Scatter of the indices of one block: ranks as in k_radix_scatter (wave
+// ballots, per-wave digit counters), written straight to their places (a
+// digit's run in a block is a few elements, so staging would not widen the
+// stores).
+template <int ITEMS>
+__global__ __launch_bounds__(RT) void k_scatter_wide(
+    const uint32_t *keys, size_t M, int keybits, int nbins,
+    const uint32_t *offs, const uint32_t *offs_chunk, int nblocks,
+    uint32_t *idx_out) {
+  extern __shared__ uint32_t lds[];
+  uint32_t *gofs = lds;                          // [nbins]
+  uint16_t *cnt = (uint16_t *)(lds + nbins);     // [NW][nbins]
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const unsigned lane = lane_id();
+  const unsigned long long below_mask =
+      lane ? (~0ull >> (64 - lane)) : 0ull;
+  const size_t c0 = (size_t)blockIdx.x * (RT * ITEMS) +
+                    (size_t)wave * (64 * ITEMS) + lane;
+  uint32_t key[ITEMS], rank[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const size_t j = c0 + (size_t)r * 64;
+    key[r] = j < M ? keys[j] : 0u;
+  }
+  for (int c = tid; c < nbins; c += RT) {
+    const size_t og = (size_t)c * nblocks + blockIdx.x;
+    gofs[c] = offs[og] + offs_chunk[og / STILE];
+  }
+  for (int c = tid; c < NW * nbins; c += RT) cnt[c] = 0;
+  __syncthreads();
+  uint16_t *mine = cnt + (size_t)wave * nbins;
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const bool valid = c0 + (size_t)r * 64 < M;
+    const unsigned long long peers = peers_of(key[r], valid, keybits);
+    const unsigned long long below = peers & below_mask;
+    const uint32_t old = mine[key[r]];
+    __builtin_amdgcn_wave_barrier();
+    if (valid && below == 0)
+      mine[key[r]] = (uint16_t)(old + (uint32_t)__popcll(peers));
+    __builtin_amdgcn_wave_barrier();
+    rank[r] = old + (uint32_t)__popcll(below);
+  }
+  __syncthreads();
+  for (int c = tid; c < nbins; c += RT) {
+    uint32_t run = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const uint32_t n = cnt[w * nbins + c];
+      cnt[w * nbins + c] = (uint16_t)run;
+      run += n;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const size_t j = c0 + (size_t)r * 64;
+    if (j < M) idx_out[gofs[key[r]] + mine[key[r]] + rank[r]] = (uint32_t)j;
+  }
 }
 
 template <typename T>
@@ -499,8 +836,9 @@ void launch_tile_subs(size_t ntiles, uint32_t *counts, uint32_t *tstart,
                       void *scanwork, hipStream_t s) {
   DMX_ASSERT(ntiles > 0, "internal: no tiles");
   if (ntiles <= (size_t)ST * TS_ITEMS) {
-    hipLaunchKernelGGL(k_tile_subs_one, dim3(1), dim3(ST), 0, s, tstart, tend,
-                       ntiles, counts, nsub, sub_start, subs, nsub_total);
+    hipLaunchKernelGGL(k_tile_subs_one, dim3(1), dim3(ST), 0, s,
+                       tstart, tend, ntiles, counts, nsub, sub_start, subs,
+                       nsub_total);
     DMX_HIP(hipGetLastError());
     return;
   }
@@ -511,6 +849,76 @@ void launch_tile_subs(size_t ntiles, uint32_t *counts, uint32_t *tstart,
                      counts, tstart, (const uint32_t *)nsub,
                      (const uint32_t *)sub_start, ntiles, subs);
   DMX_HIP(hipGetLastError());
+}
+
+bool launch_index(const Geo &g, const void *coords, size_t M, int keybits,
+                  size_t ntiles, uint32_t *idx, uint32_t *keys, void *work,
+                  uint32_t *counts, uint32_t *tstart, uint32_t *nsub,
+                  uint32_t *sub_start, Sub *subs, uint32_t *nsub_total,
+                  hipStream_t s) {
+  if (!M || ntiles > (size_t)WIDE_TILES) return false;
+#define DMX_BYDIM(KERNEL, ...)                              \
+  switch (g.ndim) {                                         \
+    case 1: KERNEL(1, __VA_ARGS__); break;                  \
+    case 2: KERNEL(2, __VA_ARGS__); break;                  \
+    default: KERNEL(3, __VA_ARGS__); break;                 \
+  }
+  if (M <= (size_t)SMALL_M) {
+#define DMX_SMALL(D, _)                                                      \
+  hipLaunchKernelGGL(k_index_small<D>, dim3(1), dim3(SMALL_T), 0, s, g,      \
+                     coords, (int)M, keybits, (int)ntiles, idx, counts,      \
+                     tstart, nsub, sub_start, subs, nsub_total)
+    DMX_BYDIM(DMX_SMALL, 0)
+#undef DMX_SMALL
+    DMX_HIP(hipGetLastError());
+    return true;
+  }
+  // blocks of 1024 points fill the chip up to about 5e5 points; the table
+  // (histogram and offsets, tiles x blocks) has to fit the workspace of the
+  // 8-bit passes, which this sort needs none of otherwise
+  const size_t room = radix_sort_workspace(M) / sizeof(uint32_t);
+  auto fits = [&](size_t items) {
+    const size_t nb = (M + RT * items - 1) / (RT * items);
+    const size_t tab = ntiles * nb;
+    return (tab + STILE - 1) / STILE <= (size_t)WIDE_CHUNKS &&
+           2 * tab + tab / STILE + 64 <= room;
+  };
+  const bool four = M <= ((size_t)1 << 19) && fits(4);
+  if (!four && !fits(16)) return false;
+  const size_t items = four ? 4 : 16;
+  const size_t nb = (M + RT * items - 1) / (RT * items), tab = ntiles * nb;
+  uint32_t *hist = (uint32_t *)work, *offs = hist + tab, *bsum = offs + tab;
+  const size_t nch = (tab + STILE - 1) / STILE;
+  const dim3 grid((unsigned)nb), block(RT);
+  const size_t lh = ntiles * 4, ls = ntiles * (4 + 2 * NW);
+#define DMX_FOLD(D, I)                                                       \
+  hipLaunchKernelGGL((k_fold_wide<D, I>), grid, block, lh, s, g, coords, M,  \
+                     keys, hist, (int)ntiles, (int)nb)
+  if (four) {
+    DMX_BYDIM(DMX_FOLD, 4)
+  } else {
+    DMX_BYDIM(DMX_FOLD, 16)
+  }
+#undef DMX_FOLD
+#undef DMX_BYDIM
+  hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nch), dim3(ST), 0, s,
+                     (const uint32_t *)hist, offs, tab, bsum);
+  hipLaunchKernelGGL(k_tiles_wide, dim3(1), dim3(1024), 0, s,
+                     (const uint32_t *)offs, bsum, (int)nch, M, (int)ntiles,
+                     (int)nb, counts, tstart, nsub, sub_start, subs,
+                     nsub_total);
+  if (four)
+    hipLaunchKernelGGL(k_scatter_wide<4>, grid, block, ls, s,
+                       (const uint32_t *)keys, M, keybits, (int)ntiles,
+                       (const uint32_t *)offs, (const uint32_t *)bsum,
+                       (int)nb, idx);
+  else
+    hipLaunchKernelGGL(k_scatter_wide<16>, grid, block, ls, s,
+                       (const uint32_t *)keys, M, keybits, (int)ntiles,
+                       (const uint32_t *)offs, (const uint32_t *)bsum,
+                       (int)nb, idx);
+  DMX_HIP(hipGetLastError());
+  return true;
 }
 
 void launch_gather_coords(const void *coords, int coord_f32, int ndim,
