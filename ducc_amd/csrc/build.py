@@ -19,7 +19,7 @@ GEN = os.path.join(HERE, "_gen")
 # the longest compilations first
 SOURCES = ["fft_f32.hip", "fft_f32_half.hip", "fft_f64.hip",
            "fft_f64_half.hip", "params.cpp", "runtime.hip", "api.hip", "sort.hip", "spread.hip",
-           "interp.hip", "fft.hip", "grid.hip", "chooser.hip", "mlp.hip",
+           "interp.hip", "interp_wave.hip", "fft.hip", "grid.hip", "chooser.hip", "mlp.hip",
            "c2c.hip", "noalloc.hip", "spread_det.hip", "records.hip",
            "sht.hip", "wgridder.hip"]
 

@@ -262,6 +262,13 @@ bool launch_index(const Geo &g, const void *coords, size_t M, int keybits,
                   uint32_t *counts, uint32_t *tstart, uint32_t *nsub,
                   uint32_t *sub_start, Sub *subs, uint32_t *nsub_total,
                   hipStream_t s);
+// subproblems of every tile's keys [k0, k1) in an order sorted by (tile, key
+// < nk); start[t * nk + k]: first position of tile t's key k (ntiles * nk + 1
+// entries)
+void launch_tiles_range(const uint32_t *start, size_t ntiles, uint32_t nk,
+                        uint32_t k0, uint32_t k1, uint32_t *nsub,
+                        uint32_t *sub_start, Sub *subs, uint32_t *nsub_total,
+                        hipStream_t s);
 void launch_gather_coords(const void *coords, int coord_f32, int ndim,
                           const uint32_t *idx, size_t M, void *out,
                           hipStream_t s);
@@ -327,6 +334,10 @@ struct SpreadArgs {
   int slab_out;
 };
 void launch_spread(bool fp64, const SpreadArgs &a, hipStream_t s);
+// 3-D FP64 interpolation with W >= 9, one wave per point (false: not a
+// request it takes, nothing launched)
+bool launch_interp_wave(const SpreadArgs &a, void *out, int out_f64,
+                        hipStream_t s);
 void launch_interp(bool fp64, const SpreadArgs &a, void *out, int out_f64,
                    hipStream_t s);
 void launch_interp_grad(bool fp64, const SpreadArgs &a, void *out,

@@ -15,6 +15,16 @@ void go(const SpreadArgs &a, void *out, int out_f64, hipStream_t s) {
     size_t cells = interp_inner_pad(a.lds_side);
     for (int d = 1; d < NDIM; ++d) cells *= a.lds_side;
     size_t sh = 2 * cells * sizeof(T);
+    // a region of more than a third of the CU's LDS: 512 threads share it
+    if constexpr (NDIM == 3) {
+      if (sh > LDS_MAX_BYTES / 3) {
+        allow_big_lds(k_interp<T, NDIM, W, true, MODE, 512>, sh);
+        hipLaunchKernelGGL((k_interp<T, NDIM, W, true, MODE, 512>), dim3(nb),
+                           dim3(512), sh, s, a, out, out_f64);
+        DMX_HIP(hipGetLastError());
+        return;
+      }
+    }
     allow_big_lds(k_interp<T, NDIM, W, true, MODE>, sh);
     hipLaunchKernelGGL((k_interp<T, NDIM, W, true, MODE>), dim3(nb), dim3(256),
                        sh, s, a, out, out_f64);
@@ -74,6 +84,7 @@ void dispatch(bool fp64, const SpreadArgs &a, void *out, int f64,
 
 void launch_interp(bool fp64, const SpreadArgs &a, void *out, int out_f64,
                    hipStream_t s) {
+  if (fp64 && launch_interp_wave(a, out, out_f64, s)) return;
   dispatch<0>(fp64, a, out, out_f64, s);
 }
 

@@ -730,9 +730,13 @@ __host__ __device__ inline int interp_inner_pad(int S) { return (S + 3) & ~1; }
 // The region is staged in LDS as interleaved complex cells (one 8/16-byte
 // read per tap); 2-D FP32 reads aligned pairs of cells (16 bytes) and picks
 // the taps by the parity of the first column.
-template <typename T, int NDIM, int W, bool LDS, int MODE>
-__global__ __launch_bounds__(256) void k_interp(SpreadArgs a, void *out,
-                                                int out_f64) {
+// NT: threads per workgroup.  A region above a third of a CU's LDS leaves
+// room for one or two workgroups: they take 512 threads, so that two waves a
+// SIMD are in flight (3-D FP64, W = 11, 104 KB regions, 1e6 clustered
+// points, before those requests went to k_interp_wave: 1400 -> 1050 us).
+template <typename T, int NDIM, int W, bool LDS, int MODE, int NT = 256>
+__global__ __launch_bounds__(NT) void k_interp(SpreadArgs a, void *out,
+                                               int out_f64) {
   using C2 = typename cplx2<T>::type;
   extern __shared__ unsigned char smem_raw[];
   const uint32_t total = *a.nsub_total;
@@ -787,11 +791,11 @@ __global__ __launch_bounds__(256) void k_interp(SpreadArgs a, void *out,
     const int part = (int)(threadIdx.x % tpp);
     const uint32_t pstep = blockDim.x / tpp;
     // one point per lane and round (tpp == 1): the indices and coordinates
-    // of all of a lane's rounds (at most MAXSUB / 256) are loaded up front,
+    // of all of a lane's rounds (at most MAXSUB / NT) are loaded up front,
     // so that their latencies overlap
     // (records: index, word and kernel arguments; the arguments are kept
     // as doubles, exact for either compute type)
-    constexpr int PF = tpp == 1 ? MAXSUB / 256 : 1;
+    constexpr int PF = tpp == 1 ? (MAXSUB + NT - 1) / NT : 1;
     uint32_t jpf[PF], wpf[PF];
     double xpf[PF][NDIM];
     if constexpr (tpp == 1) {
@@ -840,7 +844,7 @@ __global__ __launch_bounds__(256) void k_interp(SpreadArgs a, void *out,
       double x_[NDIM];
       uint32_t wd = 0;
       if constexpr (tpp == 1) {
-        // round pb / pstep (< PF: nc <= MAXSUB, pstep = 256), selected
+        // round pb / pstep (< PF: nc <= MAXSUB, pstep = NT), selected
         // with constant indices so the arrays stay in registers
         const int kk = (int)(pb / pstep);
 #pragma unroll
@@ -1042,9 +1046,9 @@ __global__ __launch_bounds__(256) void k_interp(SpreadArgs a, void *out,
     // (only for W >= 8: the extra loop variants cost registers, and smaller
     // supports come with larger oversampling, i.e. more points per tile)
     if constexpr (NDIM == 3 && MODE == 0 && W >= 8) {
-      if (nc <= 64)
+      if (nc <= NT / 4)
         point_loop(std::integral_constant<int, 4>{});
-      else if (nc <= 128)
+      else if (nc <= NT / 2)
         point_loop(std::integral_constant<int, 2>{});
       else
         point_loop(std::integral_constant<int, 1>{});
