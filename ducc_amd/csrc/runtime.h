@@ -224,6 +224,20 @@ class Plan {
   // d u2nu / d coord -> out (M, ndim) complex
   void u2nu_grad(bool forward, const void *uni, bool uni_f64,
                  const int64_t *ust, void *out, bool out_f64);
+  // Several transforms of subsets of one set of points (the w planes): the
+  // caller sorts the points once by (tile, second key) - tile_keys gives the
+  // tiles - and hands over their coordinates (float64) in that order with an
+  // identity index; each transform then takes every tile's keys [k0, k1)
+  // (launch_tiles_range; npts: the points that these are), its values and
+  // results in the sorted order.
+  void tile_keys(const void *coords, size_t M, uint32_t *keys);
+  size_t ntiles() const { return ntiles_; }
+  void use_sorted(const void *coords, size_t M, const uint32_t *identity);
+  void select_keys(const uint32_t *start, uint32_t nk, uint32_t k0,
+                   uint32_t k1, size_t npts);
+  const Sub *subs() const { return subs_.as<Sub>(); }
+  const uint32_t *nsub_total() const { return nsub_total_.as<uint32_t>(); }
+  size_t nsub_max() const { return nsub_max_; }
   // the sort results of build_index (device)
   const uint32_t *idx() const { return idx_.as<uint32_t>(); }
   uint32_t *keys_copy_to(uint32_t *dev_keys_out);  // re-fold keys
@@ -305,6 +319,7 @@ class Plan {
   static std::shared_ptr<Setup> arena_setup(const Params &p, hipStream_t s);
   std::map<int, const void *> arena_tw_;  // twiddles built in the arena
   Buf idx_, subs_, nsub_total_, sorted_coords_;
+  const uint32_t *identity_ = nullptr;  // use_sorted: points in tile order
   bool rec_ = false, rec_type1_ = false;
   RecBufs recs_{};
   Buf rec_buf_, rec_tmp_;

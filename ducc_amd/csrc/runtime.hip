@@ -754,6 +754,38 @@ void Plan::finish_index(uint32_t *counts) {
                    s_);
 }
 
+void Plan::tile_keys(const void *coords, size_t M, uint32_t *keys) {
+  Geo g = g_;
+  g.coord_f32 = 0;
+  g.coord_v2 =
+      p_.ndim == 2 && reinterpret_cast<uintptr_t>(coords) % 16 == 0 ? 1 : 0;
+  launch_fold_keys(g, coords, M, keys, nullptr, s_);
+}
+
+void Plan::use_sorted(const void *coords, size_t M,
+                      const uint32_t *identity) {
+  M_ = M;
+  coord_f32_ = false;
+  g_.coord_f32 = 0;
+  coords_ = user_coords_ = coords;
+  coords_sorted_ = true;
+  identity_ = identity;
+  g_.coord_v2 =
+      p_.ndim == 2 && reinterpret_cast<uintptr_t>(coords) % 16 == 0 ? 1 : 0;
+  tmp_tiles_.stream = s_;
+  tmp_tiles_.reset(ntiles_ * 4 * 5);
+  alloc_subs(tmp_tiles_.as<uint32_t>());
+}
+
+void Plan::select_keys(const uint32_t *start, uint32_t nk, uint32_t k0,
+                       uint32_t k1, size_t npts) {
+  Phase ph(this, "building index");
+  // (the list has room for all points, alloc_subs)
+  nsub_max_ = std::min(ntiles_, npts) + (npts + MAXSUB - 1) / MAXSUB;
+  launch_tiles_range(start, ntiles_, nk, k0, k1, tile_nsub_, tile_sub0_,
+                     subs_.as<Sub>(), nsub_total_.as<uint32_t>(), s_);
+}
+
 bool Plan::build_records(const void *coords, bool coord_f32, size_t M,
                          bool type1, const void *values, bool values_f64) {
   if (!p_.use_lds || p_.deterministic || M == 0) return false;
@@ -816,7 +848,8 @@ void Plan::fill_spread_args(SpreadArgs &a) const {
   a.g = g_;
   a.subs = subs_.as<Sub>();
   a.nsub_total = nsub_total_.as<uint32_t>();
-  a.idx = idx_.as<uint32_t>();
+  a.idx = identity_ ? identity_ : idx_.as<uint32_t>();
+  a.values_sorted = identity_ ? 1 : 0;
   a.coords = coords_;
   a.coef = su_->coef.p;
   a.nsub_max = nsub_max_;

@@ -640,6 +640,51 @@ __global__ __launch_bounds__(1024) void k_tiles_wide(
   if (tid == 0) *nsub_total = carry;
 }
 
+// Subproblems of every tile's positions [start[t * nk + k0], start[t * nk +
+// k1]) in an order sorted by (tile, second key < nk): one workgroup, four
+// consecutive tiles per thread and round.
+__global__ __launch_bounds__(1024) void k_tiles_range(
+    const uint32_t *start, size_t ntiles, uint32_t nk, uint32_t k0,
+    uint32_t k1, uint32_t *nsub, uint32_t *sstart, Sub *subs,
+    uint32_t *nsub_total) {
+  __shared__ uint32_t sh[SMALL_W];
+  constexpr int TI = 4;
+  uint32_t carry = 0, tot;
+  for (size_t c = 0; c < ntiles; c += 1024 * TI) {
+    const size_t t0 = c + (size_t)threadIdx.x * TI;
+    uint32_t a[TI], e[TI], sum = 0;
+#pragma unroll
+    for (int k = 0; k < TI; ++k) {
+      a[k] = e[k] = 0;
+      if (t0 + k < ntiles) {
+        a[k] = start[(t0 + k) * nk + k0];
+        e[k] = start[(t0 + k) * nk + k1];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < TI; ++k) sum += (e[k] - a[k] + MAXSUB - 1) / MAXSUB;
+    uint32_t ex = scan1024(sum, sh, tot) + carry;
+    carry += tot;
+#pragma unroll
+    for (int k = 0; k < TI; ++k) {
+      const uint32_t ns = (e[k] - a[k] + MAXSUB - 1) / MAXSUB;
+      if (t0 + k < ntiles) {
+        nsub[t0 + k] = ns;
+        sstart[t0 + k] = ex;
+      }
+      for (uint32_t q = 0; q < ns; ++q) {
+        Sub sb;
+        sb.tile = (uint32_t)(t0 + k);
+        sb.start = a[k] + q * MAXSUB;
+        sb.end = min(e[k], sb.start + (uint32_t)MAXSUB);
+        sb.rank = q;
+        subs[ex++] = sb;
+      }
+    }
+  }
+  if (threadIdx.x == 0) *nsub_total = carry;
+}
+
 // Scatter of the indices of one block: ranks as in k_radix_scatter (wave
 // ballots, per-wave digit counters), written straight to their places (a
 // digit's run in a block is a few elements, so staging would not widen the
@@ -919,6 +964,15 @@ bool launch_index(const Geo &g, const void *coords, size_t M, int keybits,
                        (int)nb, idx);
   DMX_HIP(hipGetLastError());
   return true;
+}
+
+void launch_tiles_range(const uint32_t *start, size_t ntiles, uint32_t nk,
+                        uint32_t k0, uint32_t k1, uint32_t *nsub,
+                        uint32_t *sub_start, Sub *subs, uint32_t *nsub_total,
+                        hipStream_t s) {
+  hipLaunchKernelGGL(k_tiles_range, dim3(1), dim3(1024), 0, s, start, ntiles,
+                     nk, k0, k1, nsub, sub_start, subs, nsub_total);
+  DMX_HIP(hipGetLastError());
 }
 
 void launch_gather_coords(const void *coords, int coord_f32, int ndim,

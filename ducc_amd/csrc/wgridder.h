@@ -38,10 +38,12 @@ struct WgPoints {
   unsigned long long *wminmax;  // ordered-key min, max of w; active count
 };
 
-// w planes: w_p = wmin + p dw, kernel support W, FP64 coefficients
+// w planes: w_p = wmin + p dw, kernel support W, FP64 coefficients; the
+// visibilities are sorted by (tile, first plane / step), nk = nplanes / step
+// keys a tile (step > 1 only where tiles * planes exceed 2^30)
 struct WgPlanes {
   double wmin, dw;
-  int nplanes, W;
+  int nplanes, W, nk, step;
   const double *coef;
 };
 
@@ -67,10 +69,11 @@ struct WgJob {
   void zero_dirty(void *dirty, bool dirty_f64, int64_t ds0, int64_t ds1);
 
  private:
-  Buf fovc_, pts_, val_, mm_, keys_, skeys_, idx_, sorted_, sval_, wcoef_;
-  std::vector<size_t> first_;
-  void sort_planes();
-  void plane_range(int p, size_t &lo, size_t &hi) const;
+  Buf fovc_, pts_, val_, mm_, idx_, ident_, start_, sorted_, sval_, wcoef_;
+  std::vector<uint32_t> per_plane_;  // visibilities by first plane
+  void sort_planes(Plan &pln);
+  // the plan's next transform takes the visibilities of plane p (false: none)
+  bool select_plane(Plan &pln, int p);
 };
 
 }  // namespace dmx

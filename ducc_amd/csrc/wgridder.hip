@@ -22,9 +22,12 @@
 // (Poisson summation; corfunc = 1 / Fourier transform of psi, the kernel's
 // correction function, wgridder.h:1361-1371), dw = 0.5 / ofactor /
 // max|m|.  Each visibility touches the W planes of its kernel support:
-// they are sorted once by first plane (stable radix sort), so every plane's
-// visibilities are one contiguous range, and each plane is one 2-D NUFFT of
-// that range with the visibilities weighted by psi, whose image is
+// they are sorted once by (uv tile, first plane) (stable radix sort), so a
+// plane's visibilities are one contiguous range of every tile, already in
+// tile order: a plane's subproblem list is one small launch, and its NUFFT
+// reads coordinates and values in sequence (an index build per plane took 75
+// us, 3.7 of 20 ms at 20000 x 64 visibilities on 25 planes).  Each plane is
+// one 2-D NUFFT with the visibilities weighted by psi, whose image is
 // multiplied by the plane's w-screen e^{-2 pi i w_p m} and accumulated
 // (gridding); degridding runs the same steps transposed.  The kernel row
 // comes from ducc0's 3-D table (as wgridder.h:1522 chooses for w-gridding):
@@ -161,22 +164,49 @@ __global__ __launch_bounds__(256) void k_wg_prep(WgArgs a, WgPoints o) {
   }
 }
 
-// first w-plane of every visibility (inactive ones: nplanes, sorted last)
-__global__ void k_wg_keys(const WgPoints o, size_t M, WgPlanes pl,
-                          uint32_t *keys) {
-  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= M) return;
-  uint32_t k = (uint32_t)pl.nplanes;
-  if (o.active[q]) {
-    const double uw = (o.w[q] - pl.wmin) / pl.dw;
-    int i0 = (int)floor(uw - 0.5 * pl.W + 1.0);
-    i0 = i0 < 0 ? 0 : (i0 > pl.nplanes - pl.W ? pl.nplanes - pl.W : i0);
-    k = (uint32_t)i0;
-  }
-  keys[q] = k;
+// first w-plane of a visibility
+__device__ __forceinline__ int first_plane(const WgPlanes &pl, double w) {
+  const double uw = (w - pl.wmin) / pl.dw;
+  const int i0 = (int)floor(uw - 0.5 * pl.W + 1.0);
+  return i0 < 0 ? 0 : (i0 > pl.nplanes - pl.W ? pl.nplanes - pl.W : i0);
 }
 
-// the visibilities in first-plane order
+// sort key of every visibility, tile * nk + first plane / step (inactive
+// ones last), the number of visibilities per key and per first plane
+constexpr int HIST_PLANES = 4096;  // planes counted in LDS
+__global__ __launch_bounds__(256) void k_wg_keys(const WgPoints o, size_t M,
+                                                 WgPlanes pl, size_t ntiles,
+                                                 uint32_t *keys,
+                                                 uint32_t *count,
+                                                 uint32_t *planes) {
+  __shared__ uint32_t h[HIST_PLANES];
+  const bool lds = pl.nplanes <= HIST_PLANES;
+  if (lds)
+    for (int c = threadIdx.x; c < pl.nplanes; c += 256) h[c] = 0;
+  __syncthreads();
+  for (size_t q = (size_t)blockIdx.x * 256 + threadIdx.x; q < M;
+       q += (size_t)gridDim.x * 256) {
+    uint32_t k = (uint32_t)(ntiles * pl.nk);
+    if (o.active[q]) {
+      const int i0 = first_plane(pl, o.w[q]);
+      k = keys[q] * pl.nk + (uint32_t)i0 / pl.step;
+      atomicAdd(&count[k], 1u);
+      atomicAdd(lds ? &h[i0] : &planes[i0], 1u);
+    }
+    keys[q] = k;
+  }
+  __syncthreads();
+  if (lds)
+    for (int c = threadIdx.x; c < pl.nplanes; c += 256)
+      if (h[c]) atomicAdd(&planes[c], h[c]);
+}
+
+__global__ void k_wg_iota(uint32_t *p, size_t n) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = (uint32_t)i;
+}
+
+// the visibilities in sorted order
 __global__ void k_wg_gather(const WgPoints o, const uint32_t *idx, size_t M,
                             WgPoints s) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -188,34 +218,41 @@ __global__ void k_wg_gather(const WgPoints o, const uint32_t *idx, size_t M,
   if (o.val) ((double2 *)s.val)[i] = ((const double2 *)o.val)[q];
 }
 
-// psi weight of plane p for the visibility at w with first plane i0
+// psi weight of plane p for the visibility at w (0 outside its planes)
 __device__ __forceinline__ double plane_weight(const WgPlanes &pl, double w,
-                                               uint32_t i0, int p) {
+                                               int p) {
+  const int q = p - first_plane(pl, w);
+  if (q < 0 || q >= pl.W) return 0.0;
   const double uw = (w - pl.wmin) / pl.dw;
-  const double frac = uw - (double)i0;
+  const double frac = uw - (double)(p - q);
   return piece_weight<double>((double)(pl.W - 1) - 2.0 * frac, pl.coef, pl.W,
-                              p - (int)i0);
+                              q);
 }
 
-// gridding, plane p: vals[i - lo] = val_s[i] * psi(w_i - w_p), in the
-// compute type (out_f64)
-__global__ void k_wg_plane_vals(const WgPoints s, const uint32_t *keys,
-                                size_t lo, size_t hi, WgPlanes pl, int p,
-                                void *vals, int out_f64) {
-  const size_t i = lo + (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= hi) return;
-  const double wt = plane_weight(pl, s.w[i], keys[i], p);
-  const double2 v = ((const double2 *)s.val)[i];
-  if (out_f64)
-    ((double2 *)vals)[i - lo] = make_double2(v.x * wt, v.y * wt);
-  else
-    ((float2 *)vals)[i - lo] =
-        make_float2((float)(v.x * wt), (float)(v.y * wt));
+// gridding, plane p: vals[i] = val_s[i] * psi(w_i - w_p) over the plane's
+// subproblems, in the compute type (out_f64)
+__global__ __launch_bounds__(256) void k_wg_plane_vals(
+    const WgPoints s, const Sub *subs, const uint32_t *nsub, WgPlanes pl,
+    int p, void *vals, int out_f64) {
+  const uint32_t n = *nsub;
+  for (uint32_t b = blockIdx.x; b < n; b += gridDim.x) {
+    const Sub sb = subs[b];
+    for (uint32_t i = sb.start + threadIdx.x; i < sb.end; i += 256) {
+      const double wt = plane_weight(pl, s.w[i], p);
+      const double2 v = ((const double2 *)s.val)[i];
+      if (out_f64)
+        ((double2 *)vals)[i] = make_double2(v.x * wt, v.y * wt);
+      else
+        ((float2 *)vals)[i] =
+            make_float2((float)(v.x * wt), (float)(v.y * wt));
+    }
+  }
 }
 
-// gridding, plane p: acc += image_p * e^{-2 pi i w_p m}
+// gridding, plane p: acc += Re(image_p * e^{-2 pi i w_p m}) (the dirty image
+// is the real part of the sum; bound by the FP64 sums' traffic)
 __global__ void k_wg_accum_image(WgArgs a, const void *img, int img_f64,
-                                 double wp, double2 *acc) {
+                                 double wp, double *acc) {
   const int i = blockIdx.y, j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= a.ny) return;
   bool inside;
@@ -228,13 +265,11 @@ __global__ void k_wg_accum_image(WgArgs a, const void *img, int img_f64,
     const float2 f = ((const float2 *)img)[k];
     z = make_double2(f.x, f.y);
   }
-  const double2 r = cmul(z, expi2pi(-wp * m));
-  acc[k].x += r.x;
-  acc[k].y += r.y;
+  acc[k] += cmul(z, expi2pi(-wp * m)).x;
 }
 
-// gridding, last step: dirty = Re(acc) * corfunc(m dw) / n (w-gridding) or
-// Re(image) (without)
+// gridding, last step: dirty = sum * corfunc(m dw) / n (w-gridding, src real
+// FP64) or Re(image) (without)
 __global__ void k_wg_finish_dirty(WgArgs a, const void *src, int src_f64,
                                   int wgrid, CorfacArgs cw, double dw,
                                   void *dirty, int dirty_f64, int64_t dst0,
@@ -242,8 +277,9 @@ __global__ void k_wg_finish_dirty(WgArgs a, const void *src, int src_f64,
   const int i = blockIdx.y, j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= a.ny) return;
   const size_t k = (size_t)i * a.ny + j;
-  double re = src_f64 ? ((const double2 *)src)[k].x
-                      : (double)((const float2 *)src)[k].x;
+  double re = wgrid ? ((const double *)src)[k]
+              : src_f64 ? ((const double2 *)src)[k].x
+                        : (double)((const float2 *)src)[k].x;
   if (wgrid) {
     bool inside;
     const double nm1 = pixel_nm1(a, i, j, inside);
@@ -308,23 +344,28 @@ __global__ void k_wg_plane_image(WgArgs a, const double *img, int wgrid,
     ((float2 *)out)[k] = make_float2((float)z.x, (float)z.y);
 }
 
-// degridding, plane p: acc_s[i] += res[i - lo] * psi(w_i - w_p)
-__global__ void k_wg_plane_accum_vis(const WgPoints s, const uint32_t *keys,
-                                     size_t lo, size_t hi, WgPlanes pl, int p,
-                                     const void *res, int res_f64,
-                                     double2 *acc) {
-  const size_t i = lo + (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= hi) return;
-  const double wt = plane_weight(pl, s.w[i], keys[i], p);
-  double2 z;
-  if (res_f64) {
-    z = ((const double2 *)res)[i - lo];
-  } else {
-    const float2 f = ((const float2 *)res)[i - lo];
-    z = make_double2(f.x, f.y);
+// degridding, plane p: acc_s[i] += res[i] * psi(w_i - w_p) over the plane's
+// subproblems
+__global__ __launch_bounds__(256) void k_wg_plane_accum_vis(
+    const WgPoints s, const Sub *subs, const uint32_t *nsub, WgPlanes pl,
+    int p, const void *res, int res_f64, double2 *acc) {
+  const uint32_t n = *nsub;
+  for (uint32_t b = blockIdx.x; b < n; b += gridDim.x) {
+    const Sub sb = subs[b];
+    for (uint32_t i = sb.start + threadIdx.x; i < sb.end; i += 256) {
+      const double wt = plane_weight(pl, s.w[i], p);
+      if (wt == 0.0) continue;
+      double2 z;
+      if (res_f64) {
+        z = ((const double2 *)res)[i];
+      } else {
+        const float2 f = ((const float2 *)res)[i];
+        z = make_double2(f.x, f.y);
+      }
+      acc[i].x += z.x * wt;
+      acc[i].y += z.y * wt;
+    }
   }
-  acc[i].x += z.x * wt;
-  acc[i].y += z.y * wt;
 }
 
 // degridding, last step: vis[row, chan] = value * wgt * e^{-2 pi i (lshift
@@ -366,6 +407,10 @@ __global__ void k_wg_finish_vis(WgArgs a, const WgPoints o, const void *res,
 }
 
 unsigned nblk(size_t n, unsigned t) { return (unsigned)((n + t - 1) / t); }
+// a workgroup per subproblem of the plane
+dim3 plane_blocks(const Plan &pln) {
+  return dim3((unsigned)std::min<size_t>(pln.nsub_max(), 8192));
+}
 double from_key(unsigned long long k) {
   const long long b = (k & 0x8000000000000000ull)
                           ? (long long)(k & 0x7FFFFFFFFFFFFFFFull)
@@ -535,22 +580,35 @@ void WgJob::choose(double eps, double smin, double smax, bool fp64_values,
   cw.W = k.W;
 }
 
-void WgJob::sort_planes() {
-  // first plane per visibility, stable sort, plane ranges
-  keys_.stream = s;
-  keys_.reset(M * 4);
-  skeys_.stream = s;
-  skeys_.reset(M * 4);
+void WgJob::sort_planes(Plan &pln) {
+  // stable sort by (tile, first plane), the start of every key
+  const size_t nt = pln.ntiles();
+  pl.step = 1;
+  auto nk = [&] { return (pl.nplanes + pl.step - 1) / pl.step; };
+  while (nt * (size_t)nk() > ((size_t)1 << 30)) pl.step *= 2;
+  pl.nk = nk();
+  const size_t ntab = nt * (size_t)pl.nk + 1;
   idx_.stream = s;
   idx_.reset(M * 4);
-  hipLaunchKernelGGL(k_wg_keys, dim3(nblk(M, 256)), dim3(256), 0, s, o, M, pl,
-                     keys_.as<uint32_t>());
+  start_.stream = s;
+  start_.reset(ntab * 4);
+  launch_zero(start_.p, start_.bytes, s);
+  Buf keys(M * 4, s), planes((size_t)pl.nplanes * 4, s);
+  launch_zero(planes.p, planes.bytes, s);
+  pln.tile_keys(o.coord, M, keys.as<uint32_t>());
+  hipLaunchKernelGGL(k_wg_keys, dim3(std::min<unsigned>(nblk(M, 256), 2048)),
+                     dim3(256), 0, s, o, M, pl, nt, keys.as<uint32_t>(),
+                     start_.as<uint32_t>(), planes.as<uint32_t>());
+  DMX_HIP(hipGetLastError());
+  Buf sw(scan_workspace(ntab), s);
+  exclusive_scan_u32(start_.as<uint32_t>(), start_.as<uint32_t>(), ntab,
+                     nullptr, sw.p, s);
   int kb = 1;
-  while ((1 << kb) <= pl.nplanes) ++kb;
+  while (((size_t)1 << kb) < ntab) ++kb;  // the largest key is ntab - 1
   const size_t ws = radix_sort_workspace(M);
   Buf work(ws, s);
-  radix_sort_pairs(keys_.as<uint32_t>(), M, kb, idx_.as<uint32_t>(),
-                   skeys_.as<uint32_t>(), work.p, ws, s);
+  radix_sort_pairs(keys.as<uint32_t>(), M, kb, idx_.as<uint32_t>(), nullptr,
+                   work.p, ws, s);
   sorted_.stream = s;
   sorted_.reset(M * 24 + 256);
   so = o;
@@ -565,25 +623,29 @@ void WgJob::sort_planes() {
   }
   hipLaunchKernelGGL(k_wg_gather, dim3(nblk(M, 256)), dim3(256), 0, s, o,
                      (const uint32_t *)idx_.p, M, so);
+  ident_.stream = s;
+  ident_.reset(M * 4);
+  hipLaunchKernelGGL(k_wg_iota, dim3(nblk(M, 256)), dim3(256), 0, s,
+                     ident_.as<uint32_t>(), M);
   DMX_HIP(hipGetLastError());
-  // visibilities per first plane -> contiguous ranges
-  std::vector<uint32_t> sk(M);
-  DMX_HIP(hipMemcpyAsync(sk.data(), skeys_.p, M * 4, hipMemcpyDeviceToHost,
-                         s));
+  pln.use_sorted(so.coord, M, ident_.as<uint32_t>());
+  // visibilities per first plane: planes without any are skipped
+  per_plane_.resize(pl.nplanes);
+  DMX_HIP(hipMemcpyAsync(per_plane_.data(), planes.p,
+                         (size_t)pl.nplanes * 4, hipMemcpyDeviceToHost, s));
   DMX_HIP(hipStreamSynchronize(s));
-  first_.assign(pl.nplanes + 2, 0);
-  // first_[k] = first sorted position with key >= k
-  size_t pos = 0;
-  for (int k = 0; k <= pl.nplanes + 1; ++k) {
-    while (pos < M && sk[pos] < (uint32_t)k) ++pos;
-    first_[k] = pos;
-  }
 }
 
-void WgJob::plane_range(int p_, size_t &lo, size_t &hi) const {
-  const int k0 = std::max(0, p_ - pl.W + 1);
-  lo = first_[k0];
-  hi = first_[std::min(p_ + 1, pl.nplanes)];
+bool WgJob::select_plane(Plan &pln, int p_) {
+  const int i0 = std::max(0, p_ - pl.W + 1);
+  const uint32_t k0 = i0 / pl.step, k1 = p_ / pl.step + 1;
+  size_t n = 0;  // of whole steps
+  for (int k = (int)(k0 * pl.step);
+       k < std::min((int)(k1 * pl.step), pl.nplanes); ++k)
+    n += per_plane_[k];
+  if (!n) return false;
+  pln.select_keys(start_.as<uint32_t>(), pl.nk, k0, k1, n);
+  return true;
 }
 
 void WgJob::grid(void *dirty, bool dirty_f64, int64_t ds0, int64_t ds1) {
@@ -604,24 +666,21 @@ void WgJob::grid(void *dirty, bool dirty_f64, int64_t ds0, int64_t ds1) {
     pln.mark_done();
     return;
   }
-  sort_planes();
-  Buf acc(nimg * 16, s), img(nimg * es, s), vals(std::max<size_t>(M, 1) * es, s);
-  launch_zero(acc.p, acc.bytes, s);
-  // one plan for all planes: each plane re-sorts its range into the plan's
+  // one plan for all planes: each plane's subproblems go to the plan's
   // buffers, which are reused in the order of the one stream
   Plan pln(p, s);
+  sort_planes(pln);
+  Buf acc(nimg * 8, s), img(nimg * es, s), vals(std::max<size_t>(M, 1) * es, s);
+  launch_zero(acc.p, acc.bytes, s);
   for (int pp = 0; pp < pl.nplanes; ++pp) {
-    size_t lo, hi;
-    plane_range(pp, lo, hi);
-    if (hi <= lo) continue;
-    hipLaunchKernelGGL(k_wg_plane_vals, dim3(nblk(hi - lo, 256)), dim3(256), 0,
-                       s, so, (const uint32_t *)skeys_.p, lo, hi, pl, pp,
-                       vals.p, p.fp64 ? 1 : 0);
-    pln.build_index(so.coord + 2 * lo, false, hi - lo, false);
+    if (!select_plane(pln, pp)) continue;
+    hipLaunchKernelGGL(k_wg_plane_vals, plane_blocks(pln), dim3(256), 0, s,
+                       so, pln.subs(), pln.nsub_total(), pl, pp, vals.p,
+                       p.fp64 ? 1 : 0);
     pln.nu2u(false, vals.p, p.fp64, img.p, p.fp64, ust);
     hipLaunchKernelGGL(k_wg_accum_image, g2, dim3(256), 0, s, a,
                        (const void *)img.p, p.fp64 ? 1 : 0,
-                       pl.wmin + pp * dw, acc.as<double2>());
+                       pl.wmin + pp * dw, acc.as<double>());
     DMX_HIP(hipGetLastError());
   }
   hipLaunchKernelGGL(k_wg_finish_dirty, g2, dim3(256), 0, s, a,
@@ -658,22 +717,19 @@ void WgJob::degrid(const void *dirty, bool dirty_f64, int64_t ds0,
     pln.mark_done();
     return;
   }
-  sort_planes();
+  Plan pln(p, s);  // one plan for all planes, as in grid()
+  sort_planes(pln);
   Buf acc(std::max<size_t>(M, 1) * 16, s), res(std::max<size_t>(M, 1) * es, s);
   launch_zero(acc.p, acc.bytes, s);
-  Plan pln(p, s);  // one plan for all planes, as in grid()
   for (int pp = 0; pp < pl.nplanes; ++pp) {
-    size_t lo, hi;
-    plane_range(pp, lo, hi);
-    if (hi <= lo) continue;
+    if (!select_plane(pln, pp)) continue;
     hipLaunchKernelGGL(k_wg_plane_image, g2, dim3(256), 0, s, a,
                        (const double *)imgd.p, 1, pl.wmin + pp * dw, img.p,
                        p.fp64 ? 1 : 0);
-    pln.build_index(so.coord + 2 * lo, false, hi - lo, false);
     pln.u2nu(true, img.p, p.fp64, ust, res.p, p.fp64);
-    hipLaunchKernelGGL(k_wg_plane_accum_vis, dim3(nblk(hi - lo, 256)),
-                       dim3(256), 0, s, so, (const uint32_t *)skeys_.p, lo, hi,
-                       pl, pp, (const void *)res.p, p.fp64 ? 1 : 0,
+    hipLaunchKernelGGL(k_wg_plane_accum_vis, plane_blocks(pln), dim3(256), 0,
+                       s, so, pln.subs(), pln.nsub_total(), pl, pp,
+                       (const void *)res.p, p.fp64 ? 1 : 0,
                        acc.as<double2>());
     DMX_HIP(hipGetLastError());
   }
