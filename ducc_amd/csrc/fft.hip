@@ -237,6 +237,7 @@ bool fft_columns_2pass(const FftLaunch &p, int L1, void *dst, bool fp64,
   int Bl = (maxel / 2 - Lm) / (Lm + 1);
   if (Bl < 32) Bl = (maxel - Lm) / (Lm + 1);
   Bl = std::min(Bl, fp64 ? 32 : 64);
+  if (Bl > (fp64 ? 8 : 16)) Bl -= Bl % (fp64 ? 8 : 16);  // whole cache lines
   Bl = std::max(1, std::min(Bl, p.nv));
   FftArgs c{};
   c.Bl = Bl;
