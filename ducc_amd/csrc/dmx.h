@@ -262,13 +262,23 @@ bool launch_index(const Geo &g, const void *coords, size_t M, int keybits,
                   uint32_t *counts, uint32_t *tstart, uint32_t *nsub,
                   uint32_t *sub_start, Sub *subs, uint32_t *nsub_total,
                   hipStream_t s);
-// subproblems of every tile's keys [k0, k1) in an order sorted by (tile, key
-// < nk); start[t * nk + k]: first position of tile t's key k (ntiles * nk + 1
-// entries)
+// subproblems of every tile's keys [k0, k1) of each range in an
+// order sorted by (tile, key < nk); start[t * nk + k]: first position of
+// tile t's key k (ntiles * nk + 1 entries).  Range r's list is at subs + r *
+// list, its tables at nsub / sub_start + r * ntiles, its length at
+// nsub_total[r].
+// At most KEY_RANGES ranges a call.
+constexpr int KEY_RANGES = 32;
+struct KeyRange {
+  uint32_t k0, k1;
+};
+struct KeyRanges {
+  KeyRange r[KEY_RANGES];
+};
 void launch_tiles_range(const uint32_t *start, size_t ntiles, uint32_t nk,
-                        uint32_t k0, uint32_t k1, uint32_t *nsub,
-                        uint32_t *sub_start, Sub *subs, uint32_t *nsub_total,
-                        hipStream_t s);
+                        const KeyRanges &ranges, size_t nranges,
+                        uint32_t *nsub, uint32_t *sub_start, Sub *subs,
+                        size_t list, uint32_t *nsub_total, hipStream_t s);
 void launch_gather_coords(const void *coords, int coord_f32, int ndim,
                           const uint32_t *idx, size_t M, void *out,
                           hipStream_t s);

@@ -227,16 +227,20 @@ class Plan {
   // Several transforms of subsets of one set of points (the w planes): the
   // caller sorts the points once by (tile, second key) - tile_keys gives the
   // tiles - and hands over their coordinates (float64) in that order with an
-  // identity index; each transform then takes every tile's keys [k0, k1)
-  // (launch_tiles_range; npts: the points that these are), its values and
-  // results in the sorted order.
+  // identity index; select_ranges builds the subproblem lists of a batch of
+  // key ranges (launch_tiles_range), and each transform takes the points of
+  // the range that use_range names, its values and results in the sorted
+  // order.
   void tile_keys(const void *coords, size_t M, uint32_t *keys);
   size_t ntiles() const { return ntiles_; }
   void use_sorted(const void *coords, size_t M, const uint32_t *identity);
-  void select_keys(const uint32_t *start, uint32_t nk, uint32_t k0,
-                   uint32_t k1, size_t npts);
-  const Sub *subs() const { return subs_.as<Sub>(); }
-  const uint32_t *nsub_total() const { return nsub_total_.as<uint32_t>(); }
+  // npts[r]: points of range r; at most KEY_RANGES ranges
+  void select_ranges(const uint32_t *start, uint32_t nk,
+                     const std::vector<KeyRange> &ranges,
+                     const std::vector<size_t> &npts);
+  void use_range(size_t r);
+  const Sub *subs() const { return cur_subs_; }
+  const uint32_t *nsub_total() const { return cur_nsub_; }
   size_t nsub_max() const { return nsub_max_; }
   // the sort results of build_index (device)
   const uint32_t *idx() const { return idx_.as<uint32_t>(); }
@@ -320,6 +324,11 @@ class Plan {
   std::map<int, const void *> arena_tw_;  // twiddles built in the arena
   Buf idx_, subs_, nsub_total_, sorted_coords_;
   const uint32_t *identity_ = nullptr;  // use_sorted: points in tile order
+  // the current subproblem list (subs_, or one range's part of it)
+  const Sub *cur_subs_ = nullptr;
+  const uint32_t *cur_nsub_ = nullptr;
+  size_t range_list_ = 0;
+  std::vector<size_t> range_nsub_;
   bool rec_ = false, rec_type1_ = false;
   RecBufs recs_{};
   Buf rec_buf_, rec_tmp_;

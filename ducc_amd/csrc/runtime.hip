@@ -744,6 +744,8 @@ void Plan::alloc_subs(uint32_t *counts) {
   subs_.reset(nsub_max_ * sizeof(Sub));
   nsub_total_.stream = s_;
   nsub_total_.reset(4);
+  cur_subs_ = subs_.as<Sub>();
+  cur_nsub_ = nsub_total_.as<uint32_t>();
 }
 
 // after the 8-bit passes: the tile table and the subproblems
@@ -772,18 +774,40 @@ void Plan::use_sorted(const void *coords, size_t M,
   identity_ = identity;
   g_.coord_v2 =
       p_.ndim == 2 && reinterpret_cast<uintptr_t>(coords) % 16 == 0 ? 1 : 0;
-  tmp_tiles_.stream = s_;
-  tmp_tiles_.reset(ntiles_ * 4 * 5);
-  alloc_subs(tmp_tiles_.as<uint32_t>());
 }
 
-void Plan::select_keys(const uint32_t *start, uint32_t nk, uint32_t k0,
-                       uint32_t k1, size_t npts) {
+void Plan::select_ranges(const uint32_t *start, uint32_t nk,
+                         const std::vector<KeyRange> &ranges,
+                         const std::vector<size_t> &npts) {
   Phase ph(this, "building index");
-  // (the list has room for all points, alloc_subs)
-  nsub_max_ = std::min(ntiles_, npts) + (npts + MAXSUB - 1) / MAXSUB;
-  launch_tiles_range(start, ntiles_, nk, k0, k1, tile_nsub_, tile_sub0_,
-                     subs_.as<Sub>(), nsub_total_.as<uint32_t>(), s_);
+  const size_t n = ranges.size();
+  range_nsub_.resize(n);
+  range_list_ = 0;
+  for (size_t r = 0; r < n; ++r) {
+    range_nsub_[r] =
+        std::min(ntiles_, npts[r]) + (npts[r] + MAXSUB - 1) / MAXSUB;
+    range_list_ = std::max(range_list_, range_nsub_[r]);
+  }
+  subs_.stream = nsub_total_.stream = tmp_tiles_.stream = s_;
+  subs_.reset(n * range_list_ * sizeof(Sub));
+  nsub_total_.reset(n * 4);
+  tmp_tiles_.reset(n * ntiles_ * 4 * 2);
+  DMX_ASSERT(n <= (size_t)KEY_RANGES, "internal: too many key ranges");
+  KeyRanges kr{};
+  std::copy(ranges.begin(), ranges.end(), kr.r);
+  launch_tiles_range(start, ntiles_, nk, kr, n,
+                     tmp_tiles_.as<uint32_t>(),
+                     tmp_tiles_.as<uint32_t>() + n * ntiles_, subs_.as<Sub>(),
+                     range_list_, nsub_total_.as<uint32_t>(), s_);
+}
+
+void Plan::use_range(size_t r) {
+  const size_t n = range_nsub_.size();
+  cur_subs_ = subs_.as<Sub>() + r * range_list_;
+  cur_nsub_ = nsub_total_.as<uint32_t>() + r;
+  tile_nsub_ = tmp_tiles_.as<uint32_t>() + r * ntiles_;
+  tile_sub0_ = tmp_tiles_.as<uint32_t>() + (n + r) * ntiles_;
+  nsub_max_ = range_nsub_[r];
 }
 
 bool Plan::build_records(const void *coords, bool coord_f32, size_t M,
@@ -846,8 +870,8 @@ uint32_t *Plan::keys_copy_to(uint32_t *dev_keys_out) {
 
 void Plan::fill_spread_args(SpreadArgs &a) const {
   a.g = g_;
-  a.subs = subs_.as<Sub>();
-  a.nsub_total = nsub_total_.as<uint32_t>();
+  a.subs = cur_subs_;
+  a.nsub_total = cur_nsub_;
   a.idx = identity_ ? identity_ : idx_.as<uint32_t>();
   a.values_sorted = identity_ ? 1 : 0;
   a.coords = coords_;

@@ -641,13 +641,19 @@ __global__ __launch_bounds__(1024) void k_tiles_wide(
 }
 
 // Subproblems of every tile's positions [start[t * nk + k0], start[t * nk +
-// k1]) in an order sorted by (tile, second key < nk): one workgroup, four
-// consecutive tiles per thread and round.
+// k1]) in an order sorted by (tile, second key < nk), for several key ranges
+// at once: one workgroup a range, four consecutive tiles per thread and
+// round (a range takes 14 us of latencies, so they run side by side).
 __global__ __launch_bounds__(1024) void k_tiles_range(
-    const uint32_t *start, size_t ntiles, uint32_t nk, uint32_t k0,
-    uint32_t k1, uint32_t *nsub, uint32_t *sstart, Sub *subs,
+    const uint32_t *start, size_t ntiles, uint32_t nk, KeyRanges ranges,
+    uint32_t *nsub, uint32_t *sstart, Sub *subs, size_t list,
     uint32_t *nsub_total) {
   __shared__ uint32_t sh[SMALL_W];
+  const uint32_t k0 = ranges.r[blockIdx.x].k0, k1 = ranges.r[blockIdx.x].k1;
+  nsub += blockIdx.x * ntiles;
+  sstart += blockIdx.x * ntiles;
+  subs += blockIdx.x * list;
+  nsub_total += blockIdx.x;
   constexpr int TI = 4;
   uint32_t carry = 0, tot;
   for (size_t c = 0; c < ntiles; c += 1024 * TI) {
@@ -967,11 +973,13 @@ bool launch_index(const Geo &g, const void *coords, size_t M, int keybits,
 }
 
 void launch_tiles_range(const uint32_t *start, size_t ntiles, uint32_t nk,
-                        uint32_t k0, uint32_t k1, uint32_t *nsub,
-                        uint32_t *sub_start, Sub *subs, uint32_t *nsub_total,
-                        hipStream_t s) {
-  hipLaunchKernelGGL(k_tiles_range, dim3(1), dim3(1024), 0, s, start, ntiles,
-                     nk, k0, k1, nsub, sub_start, subs, nsub_total);
+                        const KeyRanges &ranges, size_t nranges,
+                        uint32_t *nsub, uint32_t *sub_start, Sub *subs,
+                        size_t list, uint32_t *nsub_total, hipStream_t s) {
+  DMX_ASSERT(nranges <= (size_t)KEY_RANGES, "internal: too many key ranges");
+  hipLaunchKernelGGL(k_tiles_range, dim3((unsigned)nranges), dim3(1024), 0, s,
+                     start, ntiles, nk, ranges, nsub, sub_start, subs, list,
+                     nsub_total);
   DMX_HIP(hipGetLastError());
 }
 

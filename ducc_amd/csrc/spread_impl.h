@@ -653,10 +653,32 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
             atomicAdd(&grid[2 * gi], (T)__builtin_nanf(""));
           }
         }
+        // A tile with one subproblem alone reaches the cells at offsets
+        // [W-1, tile) of its region (its neighbours' regions overlap the
+        // rest, and the periodic wrap brings other tiles' points only to the
+        // first and last nsafe cells of the grid): plain stores onto the
+        // zeroed grid there, atomics elsewhere.  64 x 64 tiles, W = 7: 69 %
+        // of the cells, 93 -> 84 us per w plane of 3.6e5 points on 3750^2
+        // cells.
+        auto mine = [&](int o, int d, int n) {
+          return o >= W - 1 && o < tile &&
+                 (unsigned)(b0[d] + o - a.g.nsafe) <
+                     (unsigned)max(n - 2 * a.g.nsafe, 0);
+        };
+        auto flush = [&](auto single_c) {
+        constexpr bool SINGLE = decltype(single_c)::value;
         RegionWalk<NDIM> rw = flush_walk0;
         for (int c = tid; c < ncell && !(FIX && fbad); c += blockDim.x) {
           // this cell's grid element, then the lane's next cell
           const size_t gi = region_grid_index(rw, b0, n0, n1, n2);
+          bool own = SINGLE;
+          if constexpr (!SINGLE) {
+          } else if constexpr (NDIM == 1) own = mine(rw.w, 0, n0);
+          else if constexpr (NDIM == 2)
+            own = mine(rw.u, 0, n0) && mine(rw.w, 1, n1);
+          else
+            own = mine(rw.u, 0, n0) && mine(rw.v, 1, n1) &&
+                  mine(rw.w, 2, n2);
           rw.next();
           T re, im;
           if constexpr (FIX) {
@@ -671,9 +693,22 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
             im = (T)sim[c];
           }
           if (re == T(0) && im == T(0)) continue;
-          atomicAdd(&grid[2 * gi], re);
-          atomicAdd(&grid[2 * gi + 1], im);
+          if (own) {
+            typename cplx2<T>::type v;
+            v.x = re;
+            v.y = im;
+            ((typename cplx2<T>::type *)grid)[gi] = v;
+          } else {
+            atomicAdd(&grid[2 * gi], re);
+            atomicAdd(&grid[2 * gi + 1], im);
+          }
         }
+        };
+        // (the test costs crowded tiles, which have several subproblems, 2 %)
+        if (a.tile_nsub[sb.tile] == 1)
+          flush(std::integral_constant<bool, true>{});
+        else
+          flush(std::integral_constant<bool, false>{});
         __syncthreads();
       } else {
         // direct HBM accumulation with periodic wrap (regions beyond LDS)

@@ -72,8 +72,7 @@ struct WgJob {
   Buf fovc_, pts_, val_, mm_, idx_, ident_, start_, sorted_, sval_, wcoef_;
   std::vector<uint32_t> per_plane_;  // visibilities by first plane
   void sort_planes(Plan &pln);
-  // the plan's next transform takes the visibilities of plane p (false: none)
-  bool select_plane(Plan &pln, int p);
+  std::vector<int> select_planes(Plan &pln, int &p);
 };
 
 }  // namespace dmx

@@ -636,16 +636,27 @@ void WgJob::sort_planes(Plan &pln) {
   DMX_HIP(hipStreamSynchronize(s));
 }
 
-bool WgJob::select_plane(Plan &pln, int p_) {
-  const int i0 = std::max(0, p_ - pl.W + 1);
-  const uint32_t k0 = i0 / pl.step, k1 = p_ / pl.step + 1;
-  size_t n = 0;  // of whole steps
-  for (int k = (int)(k0 * pl.step);
-       k < std::min((int)(k1 * pl.step), pl.nplanes); ++k)
-    n += per_plane_[k];
-  if (!n) return false;
-  pln.select_keys(start_.as<uint32_t>(), pl.nk, k0, k1, n);
-  return true;
+// the subproblem lists of the next planes from p_ on (as many as KEY_RANGES
+// that have visibilities); returns those planes
+std::vector<int> WgJob::select_planes(Plan &pln, int &p_) {
+  std::vector<int> planes;
+  std::vector<KeyRange> kr;
+  std::vector<size_t> np;
+  for (; p_ < pl.nplanes && planes.size() < (size_t)KEY_RANGES; ++p_) {
+    const int i0 = std::max(0, p_ - pl.W + 1);
+    const uint32_t k0 = i0 / pl.step, k1 = p_ / pl.step + 1;
+    size_t n = 0;  // of whole steps
+    for (int k = (int)(k0 * pl.step);
+         k < std::min((int)(k1 * pl.step), pl.nplanes); ++k)
+      n += per_plane_[k];
+    if (!n) continue;
+    planes.push_back(p_);
+    kr.push_back({k0, k1});
+    np.push_back(n);
+  }
+  if (!planes.empty())
+    pln.select_ranges(start_.as<uint32_t>(), pl.nk, kr, np);
+  return planes;
 }
 
 void WgJob::grid(void *dirty, bool dirty_f64, int64_t ds0, int64_t ds1) {
@@ -672,16 +683,20 @@ void WgJob::grid(void *dirty, bool dirty_f64, int64_t ds0, int64_t ds1) {
   sort_planes(pln);
   Buf acc(nimg * 8, s), img(nimg * es, s), vals(std::max<size_t>(M, 1) * es, s);
   launch_zero(acc.p, acc.bytes, s);
-  for (int pp = 0; pp < pl.nplanes; ++pp) {
-    if (!select_plane(pln, pp)) continue;
-    hipLaunchKernelGGL(k_wg_plane_vals, plane_blocks(pln), dim3(256), 0, s,
-                       so, pln.subs(), pln.nsub_total(), pl, pp, vals.p,
-                       p.fp64 ? 1 : 0);
-    pln.nu2u(false, vals.p, p.fp64, img.p, p.fp64, ust);
-    hipLaunchKernelGGL(k_wg_accum_image, g2, dim3(256), 0, s, a,
-                       (const void *)img.p, p.fp64 ? 1 : 0,
-                       pl.wmin + pp * dw, acc.as<double>());
-    DMX_HIP(hipGetLastError());
+  for (int next = 0; next < pl.nplanes;) {
+    const std::vector<int> planes = select_planes(pln, next);
+    for (size_t r = 0; r < planes.size(); ++r) {
+      const int pp = planes[r];
+      pln.use_range(r);
+      hipLaunchKernelGGL(k_wg_plane_vals, plane_blocks(pln), dim3(256), 0, s,
+                         so, pln.subs(), pln.nsub_total(), pl, pp, vals.p,
+                         p.fp64 ? 1 : 0);
+      pln.nu2u(false, vals.p, p.fp64, img.p, p.fp64, ust);
+      hipLaunchKernelGGL(k_wg_accum_image, g2, dim3(256), 0, s, a,
+                         (const void *)img.p, p.fp64 ? 1 : 0,
+                         pl.wmin + pp * dw, acc.as<double>());
+      DMX_HIP(hipGetLastError());
+    }
   }
   hipLaunchKernelGGL(k_wg_finish_dirty, g2, dim3(256), 0, s, a,
                      (const void *)acc.p, 1, 1, cw, dw, dirty,
@@ -721,17 +736,21 @@ void WgJob::degrid(const void *dirty, bool dirty_f64, int64_t ds0,
   sort_planes(pln);
   Buf acc(std::max<size_t>(M, 1) * 16, s), res(std::max<size_t>(M, 1) * es, s);
   launch_zero(acc.p, acc.bytes, s);
-  for (int pp = 0; pp < pl.nplanes; ++pp) {
-    if (!select_plane(pln, pp)) continue;
-    hipLaunchKernelGGL(k_wg_plane_image, g2, dim3(256), 0, s, a,
-                       (const double *)imgd.p, 1, pl.wmin + pp * dw, img.p,
-                       p.fp64 ? 1 : 0);
-    pln.u2nu(true, img.p, p.fp64, ust, res.p, p.fp64);
-    hipLaunchKernelGGL(k_wg_plane_accum_vis, plane_blocks(pln), dim3(256), 0,
-                       s, so, pln.subs(), pln.nsub_total(), pl, pp,
-                       (const void *)res.p, p.fp64 ? 1 : 0,
-                       acc.as<double2>());
-    DMX_HIP(hipGetLastError());
+  for (int next = 0; next < pl.nplanes;) {
+    const std::vector<int> planes = select_planes(pln, next);
+    for (size_t r = 0; r < planes.size(); ++r) {
+      const int pp = planes[r];
+      pln.use_range(r);
+      hipLaunchKernelGGL(k_wg_plane_image, g2, dim3(256), 0, s, a,
+                         (const double *)imgd.p, 1, pl.wmin + pp * dw, img.p,
+                         p.fp64 ? 1 : 0);
+      pln.u2nu(true, img.p, p.fp64, ust, res.p, p.fp64);
+      hipLaunchKernelGGL(k_wg_plane_accum_vis, plane_blocks(pln), dim3(256), 0,
+                         s, so, pln.subs(), pln.nsub_total(), pl, pp,
+                         (const void *)res.p, p.fp64 ? 1 : 0,
+                         acc.as<double2>());
+      DMX_HIP(hipGetLastError());
+    }
   }
   hipLaunchKernelGGL(k_wg_finish_vis, dim3(nblk(M, 256)), dim3(256), 0, s, a,
                      o, (const void *)acc.p, 1, (const uint32_t *)idx_.p, M,
