@@ -24,6 +24,15 @@ void go(const SpreadArgs &a, hipStream_t s) {
       const size_t shf =
           fix_region_bytes(cells) + sizeof(SpreadStash<T, NDIM, true>);
       if (a.fixacc && shf <= LDS_MAX_BYTES) {
+        if constexpr (NDIM == 2) {
+          if (a.coords_sorted) {
+            allow_big_lds(k_spread<T, NDIM, W, true, true, 512>, shf);
+            hipLaunchKernelGGL((k_spread<T, NDIM, W, true, true, 512>),
+                               dim3(nb), dim3(512), shf, s, a);
+            DMX_HIP(hipGetLastError());
+            return;
+          }
+        }
         allow_big_lds(k_spread<T, NDIM, W, true, true>, shf);
         hipLaunchKernelGGL((k_spread<T, NDIM, W, true, true>), dim3(nb),
                            dim3(256), shf, s, a);

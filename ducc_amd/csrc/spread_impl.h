@@ -166,7 +166,7 @@ __device__ __forceinline__ void spread_row3(Acc *sre, Acc *sim, int row,
 // quarter-wave: 16 lanes whose cells are distinct mod 16 run at ~7 lane-
 // atomics/CU/clock, random cells at ~2.5 (measured on gfx950), and these
 // atomics bound the spreader.  So:
-// phase 1 (thread t <-> points t, t+256, ... of the chunk, all loads in
+// phase 1 (thread t <-> points t, t+NT, ... of the chunk, all loads in
 //   flight first): fold, kernel argument, region offset and value; a rank
 //   inside the point's class (first cell mod 16); after a prefix over the 16
 //   classes each point has a position in the class-sorted order, which is
@@ -260,8 +260,15 @@ __device__ __forceinline__ int region_cell(uint32_t o, int S) {
   else return (o0 * S + o1) * S + o2;
 }
 
-template <typename T, int NDIM, int W, bool LDS, bool FIX = false>
-__global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
+// NT threads: 256, or 512 for points stored in tile order (2-D fixed point:
+// plans, w planes).  Those wait for nothing long, and eight waves shorten
+// each step of a subproblem (81 -> 71 us per w plane, 83 -> 77 us in a plan
+// of 1.5e6 points); gathered points want more independent workgroups instead
+// (1e7 clustered points: 475 us with 256 threads, 520 us with 512).
+template <typename T, int NDIM, int W, bool LDS, bool FIX = false,
+          int NT = 256>
+__global__ __launch_bounds__(NT) void k_spread(SpreadArgs a) {
+  constexpr int NWV = NT / 64;
   static_assert(!FIX || (sizeof(T) == 4 && LDS), "fixed point: FP32 in LDS");
   extern __shared__ unsigned char smem_raw[];
   const uint32_t total = *a.nsub_total;
@@ -287,7 +294,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
   const T *cf = (const T *)a.coef;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // the flush's walk over the region (sides S), split once per lane
-  const RegionWalk<NDIM> flush_walk0(tid, (int)blockDim.x, S, S);
+  const RegionWalk<NDIM> flush_walk0(tid, NT, S, S);
   for (uint32_t sidx0 = blockIdx.x; sidx0 < total; sidx0 += gridDim.x) {
     // stored regions: a tile's first subproblem brings all of the tile's
     // subproblems to this workgroup, the others are skipped
@@ -303,7 +310,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
       int b0[3];
       tile_origin(a.g, sb.tile, b0);
       if constexpr (LDS) {
-        for (int c = tid; c < ncell; c += blockDim.x) {
+        for (int c = tid; c < ncell; c += NT) {
           if constexpr (FIX) {
             sfx[c] = 0ull;
           } else {
@@ -313,7 +320,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
         }
         float fscale = 1.f, finv = 1.f;  // FIX: this subproblem's scale
         bool fbad = false;  // FIX: a value of the subproblem is not finite
-        constexpr int SC = SpreadStash<T, NDIM, FIX>::SC, PT = SC / 256;
+        constexpr int SC = SpreadStash<T, NDIM, FIX>::SC, PT = SC / NT;
         for (uint32_t c0 = sb.start; c0 < sb.end; c0 += SC) {
           const int nc = (int)min((uint32_t)SC, sb.end - c0);
           const int K = (nc + 63) >> 6;            // run length
@@ -341,7 +348,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
             const uint32_t tm = (1u << L) - 1u;
 #pragma unroll
             for (int k = 0; k < PT; ++k) {
-              const int i = tid + 256 * k;
+              const int i = tid + NT * k;
               os[k] = 0;
               if (i < nc) {
                 const uint32_t p = c0 + i;
@@ -366,12 +373,12 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
             double cc[PT][NDIM];
 #pragma unroll
             for (int k = 0; k < PT; ++k) {
-              const int i = tid + 256 * k;
+              const int i = tid + NT * k;
               jj[k] = i < nc ? a.idx[c0 + i] : 0u;
             }
 #pragma unroll
             for (int k = 0; k < PT; ++k) {
-              const int i = tid + 256 * k;
+              const int i = tid + NT * k;
               if (i < nc) {
                 const uint32_t p = c0 + i;
                 const size_t cj = a.coords_sorted ? (size_t)p : (size_t)jj[k];
@@ -383,7 +390,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
             }
 #pragma unroll
             for (int k = 0; k < PT; ++k) {
-              const int i = tid + 256 * k;
+              const int i = tid + NT * k;
               os[k] = 0;
               if (i < nc) {
                 uint32_t o = 0;
@@ -405,7 +412,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
           }
 #pragma unroll
           for (int k = 0; k < PT; ++k) {
-            const int i = tid + 256 * k;
+            const int i = tid + NT * k;
             cls[k] = 0;
             rnk[k] = 0;
             if (i < nc) {
@@ -419,7 +426,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
 #pragma unroll
             for (int k = 0; k < PT; ++k) {
               amax[k] = 0.f;
-              if (tid + 256 * k < nc) {
+              if (tid + NT * k < nc) {
                 const float ar = fabsf((float)vr_[k]),
                             ai = fabsf((float)vi_[k]);
                 // fmaxf ignores NaN: a NaN part counts as infinite
@@ -446,7 +453,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
             if (nblk <= FIX_MAXBLK && vmax > 0.f) {
 #pragma unroll
               for (int k = 0; k < PT; ++k) {
-                if (tid + 256 * k >= nc) continue;
+                if (tid + NT * k >= nc) continue;
                 const uint32_t q =
                     (uint32_t)ceilf(amax[k] / vmax * 1048576.f);
                 int blo[3] = {0, 0, 0}, bhi[3] = {0, 0, 0};
@@ -497,7 +504,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
           }
 #pragma unroll
           for (int k = 0; k < PT; ++k) {
-            const int i = tid + 256 * k;
+            const int i = tid + NT * k;
             if (i < nc) {
               const uint32_t pos = st.off[cls[k]] + rnk[k];
               const uint32_t r = (pos * kmul) >> 16, jr = pos - r * K;
@@ -516,13 +523,14 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
             fbad = !(__uint_as_float(fx.vmaxb) <= 3.4028235e38f);
           }
           const int run = ((lane & 15) << 2) | (lane >> 4);
-          // 3-D tiles of few points (runs shorter than the four waves): every
-          // wave takes every run and a quarter of each point's W planes, so
+          // 3-D tiles of few points (runs shorter than the waves): every
+          // wave takes every run and a share of each point's W planes, so
           // all waves work; the planes shift all lanes alike, which keeps
           // the lanes of a quarter-wave on distinct classes
-          const bool split = NDIM == 3 && K < 4;
-          const int jr0 = split ? 0 : wave, jstep = split ? 1 : 4;
-          const int q00 = split ? wave : 0, qstep = split ? 4 : 1;
+          const bool split = NDIM == 3 && K * ((W + NWV - 1) / NWV) <
+                                             (K + NWV - 1) / NWV * W;
+          const int jr0 = split ? 0 : wave, jstep = split ? 1 : NWV;
+          const int q00 = split ? wave : 0, qstep = split ? NWV : 1;
           for (int jr = jr0; jr < K; jr += jstep) {
             if (run * K + jr >= nc) continue;
             const int i = jr * 64 + run;
@@ -615,7 +623,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
           // non-finite value makes every cell NaN.
           typename cplx2<T>::type *dst =
               (typename cplx2<T>::type *)a.slab + (size_t)sb.tile * ncell;
-          for (int c = tid; c < ncell; c += blockDim.x) {
+          for (int c = tid; c < ncell; c += NT) {
             T re, im;
             if constexpr (FIX) {
               int ri, ii;
@@ -668,7 +676,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
         auto flush = [&](auto single_c) {
         constexpr bool SINGLE = decltype(single_c)::value;
         RegionWalk<NDIM> rw = flush_walk0;
-        for (int c = tid; c < ncell && !(FIX && fbad); c += blockDim.x) {
+        for (int c = tid; c < ncell && !(FIX && fbad); c += NT) {
           // this cell's grid element, then the lane's next cell
           const size_t gi = region_grid_index(rw, b0, n0, n1, n2);
           bool own = SINGLE;
@@ -714,7 +722,7 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs a) {
         // direct HBM accumulation with periodic wrap (regions beyond LDS)
         const int n0 = a.g.nover[0], n1 = NDIM > 1 ? a.g.nover[1] : 1,
                   n2 = NDIM > 2 ? a.g.nover[2] : 1;
-        for (uint32_t p = sb.start + tid; p < sb.end; p += blockDim.x) {
+        for (uint32_t p = sb.start + tid; p < sb.end; p += NT) {
           uint32_t j;
           int i0[3];
           T w[NDIM][W];
