@@ -523,15 +523,28 @@ __global__ __launch_bounds__(NT) void k_spread(SpreadArgs a) {
             fbad = !(__uint_as_float(fx.vmaxb) <= 3.4028235e38f);
           }
           const int run = ((lane & 15) << 2) | (lane >> 4);
-          // 3-D tiles of few points (runs shorter than the waves): every
-          // wave takes every run and a share of each point's W planes, so
-          // all waves work; the planes shift all lanes alike, which keeps
-          // the lanes of a quarter-wave on distinct classes
-          const bool split = NDIM == 3 && K * ((W + NWV - 1) / NWV) <
-                                             (K + NWV - 1) / NWV * W;
-          const int jr0 = split ? 0 : wave, jstep = split ? 1 : NWV;
-          const int q00 = split ? wave : 0, qstep = split ? NWV : 1;
-          for (int jr = jr0; jr < K; jr += jstep) {
+          // 3-D: a run's W planes may be dealt to 2 or 4 waves, so that few
+          // runs keep all waves busy (the planes shift all lanes alike, which
+          // keeps the lanes of a quarter-wave on distinct classes).  The
+          // split f with the least rounds * (planes + 1), the one for the
+          // point's weights: 5 runs (300 points a tile) take 12 instead of
+          // 14 on four waves.
+          int fl = 0;  // log2 f
+          if constexpr (NDIM == 3) {
+            int best = 1 << 30;
+#pragma unroll
+            for (int l = 0; l < 3; ++l) {
+              const int cost = ((K << l) + NWV - 1) / NWV *
+                               ((W + (1 << l) - 1) / (1 << l) + 1);
+              if (cost < best) {
+                best = cost;
+                fl = l;
+              }
+            }
+          }
+          const int qstep = 1 << fl;
+          for (int n = wave; n < K << fl; n += NWV) {
+            const int jr = n >> fl, q00 = n & (qstep - 1);
             if (run * K + jr >= nc) continue;
             const int i = jr * 64 + run;
             const uint32_t o = st.o[i];
