@@ -559,7 +559,7 @@ __global__ __launch_bounds__(SMALL_T) void k_index_small(
 // and subproblems, scatter: four launches and one trip of the points where
 // the 8-bit passes take ten launches and two.  1e6 points in 364 tiles:
 // 62 -> 39 us; 1e5 points in 289 tiles: 60 -> 21 us; 2e6 points in 1600
-// tiles: 87 -> 69 us.
+// tiles: 87 -> 61 us.
 constexpr int WIDE_TILES = 4096;
 
 template <int NDIM, int ITEMS>
@@ -692,23 +692,29 @@ __global__ __launch_bounds__(1024) void k_tiles_range(
 }
 
 // Scatter of the indices of one block: ranks as in k_radix_scatter (wave
-// ballots, per-wave digit counters), written straight to their places (a
-// digit's run in a block is a few elements, so staging would not widen the
-// stores).
+// ballots, per-wave digit counters).  Blocks of 4096 points (ITEMS 16) stage
+// the indices in tile order in LDS, so that a tile's run in the block goes
+// out as one piece: what bounds the scatter is the number of separate stores
+// (2e6 points in 1600 tiles, runs of 2.6: 28 us, 36 us without staging).
+// Blocks of 1024 points have runs of about one and store directly.
 template <int ITEMS>
 __global__ __launch_bounds__(RT) void k_scatter_wide(
     const uint32_t *keys, size_t M, int keybits, int nbins,
     const uint32_t *offs, const uint32_t *offs_chunk, int nblocks,
     uint32_t *idx_out) {
+  constexpr bool STAGE = ITEMS == 16;
   extern __shared__ uint32_t lds[];
-  uint32_t *gofs = lds;                          // [nbins]
-  uint16_t *cnt = (uint16_t *)(lds + nbins);     // [NW][nbins]
+  uint32_t *sh = lds;                               // [RT] (scan)
+  uint32_t *gofs = lds + RT;                        // [nbins]
+  uint32_t *sidx = gofs + nbins;                    // [RT * ITEMS] (STAGE)
+  uint16_t *cnt = (uint16_t *)(sidx + (STAGE ? RT * ITEMS : 0));  // [NW][nbins]
+  uint16_t *skey = cnt + (size_t)NW * nbins;        // [RT * ITEMS] (STAGE)
   const int tid = threadIdx.x, wave = tid >> 6;
   const unsigned lane = lane_id();
   const unsigned long long below_mask =
       lane ? (~0ull >> (64 - lane)) : 0ull;
-  const size_t c0 = (size_t)blockIdx.x * (RT * ITEMS) +
-                    (size_t)wave * (64 * ITEMS) + lane;
+  const size_t blk0 = (size_t)blockIdx.x * (RT * ITEMS);
+  const size_t c0 = blk0 + (size_t)wave * (64 * ITEMS) + lane;
   uint32_t key[ITEMS], rank[ITEMS];
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
@@ -735,20 +741,56 @@ __global__ __launch_bounds__(RT) void k_scatter_wide(
     rank[r] = old + (uint32_t)__popcll(below);
   }
   __syncthreads();
-  for (int c = tid; c < nbins; c += RT) {
-    uint32_t run = 0;
+  // per tile: the waves' prefixes (and, staged, its start in the block)
+  if constexpr (STAGE) {
+    const int per = (nbins + RT - 1) / RT, d0 = tid * per,
+              d1 = min(d0 + per, nbins);
+    uint32_t sum = 0, tot;
+    for (int c = d0; c < d1; ++c)
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const uint32_t n = cnt[w * nbins + c];
-      cnt[w * nbins + c] = (uint16_t)run;
-      run += n;
+      for (int w = 0; w < NW; ++w) sum += cnt[w * nbins + c];
+    uint32_t run = block_exclusive_scan(sum, sh, tot);
+    for (int c = d0; c < d1; ++c) {
+      gofs[c] -= run;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const uint32_t n = cnt[w * nbins + c];
+        cnt[w * nbins + c] = (uint16_t)run;
+        run += n;
+      }
+    }
+  } else {
+    for (int c = tid; c < nbins; c += RT) {
+      uint32_t run = 0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const uint32_t n = cnt[w * nbins + c];
+        cnt[w * nbins + c] = (uint16_t)run;
+        run += n;
+      }
     }
   }
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
     const size_t j = c0 + (size_t)r * 64;
-    if (j < M) idx_out[gofs[key[r]] + mine[key[r]] + rank[r]] = (uint32_t)j;
+    if (j >= M) continue;
+    const uint32_t p = mine[key[r]] + rank[r];
+    if constexpr (STAGE) {
+      sidx[p] = (uint32_t)j;
+      skey[p] = (uint16_t)key[r];
+    } else {
+      idx_out[gofs[key[r]] + p] = (uint32_t)j;
+    }
+  }
+  if constexpr (STAGE) {
+    __syncthreads();
+    const int n = (int)min((size_t)(RT * ITEMS), M - blk0);
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int q = i * RT + tid;
+      if (q < n) idx_out[gofs[skey[q]] + (uint32_t)q] = sidx[q];
+    }
   }
 }
 
@@ -941,7 +983,7 @@ bool launch_index(const Geo &g, const void *coords, size_t M, int keybits,
   uint32_t *hist = (uint32_t *)work, *offs = hist + tab, *bsum = offs + tab;
   const size_t nch = (tab + STILE - 1) / STILE;
   const dim3 grid((unsigned)nb), block(RT);
-  const size_t lh = ntiles * 4, ls = ntiles * (4 + 2 * NW);
+  const size_t lh = ntiles * 4, ls = RT * 4 + ntiles * (4 + 2 * NW);
 #define DMX_FOLD(D, I)                                                       \
   hipLaunchKernelGGL((k_fold_wide<D, I>), grid, block, lh, s, g, coords, M,  \
                      keys, hist, (int)ntiles, (int)nb)
@@ -963,11 +1005,14 @@ bool launch_index(const Geo &g, const void *coords, size_t M, int keybits,
                        (const uint32_t *)keys, M, keybits, (int)ntiles,
                        (const uint32_t *)offs, (const uint32_t *)bsum,
                        (int)nb, idx);
-  else
-    hipLaunchKernelGGL(k_scatter_wide<16>, grid, block, ls, s,
+  else {
+    const size_t lst = ls + (size_t)RT * 16 * (4 + 2);  // the staged block
+    allow_big_lds(k_scatter_wide<16>, lst);
+    hipLaunchKernelGGL(k_scatter_wide<16>, grid, block, lst, s,
                        (const uint32_t *)keys, M, keybits, (int)ntiles,
                        (const uint32_t *)offs, (const uint32_t *)bsum,
                        (int)nb, idx);
+  }
   DMX_HIP(hipGetLastError());
   return true;
 }
