@@ -293,6 +293,11 @@ __global__ __launch_bounds__(NT) void k_spread(SpreadArgs a) {
   T *grid = (T *)a.grid;
   const T *cf = (const T *)a.coef;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // cells of a region that no other tile's points reach: more than half?
+  int nown = max(tile - W + 1, 0);
+  if (NDIM > 1) nown *= max(tile - W + 1, 0);
+  if (NDIM > 2) nown *= max(tile - W + 1, 0);
+  const bool mostly_own = 2 * nown > ncell;
   // the flush's walk over the region (sides S), split once per lane
   const RegionWalk<NDIM> flush_walk0(tid, NT, S, S);
   for (uint32_t sidx0 = blockIdx.x; sidx0 < total; sidx0 += gridDim.x) {
@@ -725,8 +730,9 @@ __global__ __launch_bounds__(NT) void k_spread(SpreadArgs a) {
           }
         }
         };
-        // (the test costs crowded tiles, which have several subproblems, 2 %)
-        if (a.tile_nsub[sb.tile] == 1)
+        // (only where these are most of the region's cells: at less, or in
+        // crowded tiles with several subproblems, the test costs 2-5 %)
+        if (mostly_own && a.tile_nsub[sb.tile] == 1)
           flush(std::integral_constant<bool, true>{});
         else
           flush(std::integral_constant<bool, false>{});
