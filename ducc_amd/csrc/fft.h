@@ -35,7 +35,7 @@ struct FftPass {
 struct FftLaunch {
   void *data;       // result (and input, in place)
   const void *src;  // input at the same positions (null: data)
-  double scale;     // the input's factor (0: one)
+  double scale = 1.0;  // the input's factor
   const void *tw;  // exp(-2 pi i m / L), m < L, compute type
   int L, npass, sign;
   FftPass pass[FFT_MAXPASS];
@@ -74,7 +74,7 @@ struct FftArgs {
   void *dst;
   const void *tw;       // twiddles of length Ls
   const void *tw_full;  // twiddles of length L (twiddle)
-  double scale;         // factor of the input
+  double scale = 1.0;   // factor of the input
   int Ls, LP, Bl, npass;
   FftPass pass[FFT_MAXPASS];
   int nv, vn1, va1, va2;

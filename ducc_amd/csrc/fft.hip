@@ -147,7 +147,6 @@ void launch_fft(FftArgs &a, bool fp64, int sign, unsigned ny, unsigned nz,
   const int nel = a.Bl * a.Ls;
   const bool half = nel <= full / 2;
   a.LP = a.Bl > 1 ? a.Ls | 1 : a.Ls;
-  if (a.scale == 0.0) a.scale = 1.0;
   a.npass = plan_passes(a.Ls, radices_for(half ? full / 2 : full, nel),
                         a.pass);
   const size_t sh = ((size_t)a.Bl * a.LP + (a.tw_lds ? a.Ls : 0)) *
@@ -432,7 +431,6 @@ void fft_lineset(const FftLaunch &base, bool fp64, void *scratch,
   };
   // out of place: start so that the last pass writes the data array
   if (src != p.data && p.npass % 2 == 1) dst = p.data;
-  if (p.scale == 0.0) p.scale = 1.0;
   for (int i = 0; i < p.npass; ++i) {
     run(p.pass[i].radix);
     Ns *= p.pass[i].radix;

@@ -1,11 +1,13 @@
 """GPU: the FFT passes at their edges - every radix alone and combined, line
 counts that leave a workgroup partly filled, lines that take two passes over
 L1 x L2, out-of-place input with a factor - against a 64-bit FFT."""
+import ctypes as ct
+
 import numpy as np
 import pytest
 import torch
 
-from ducc_amd import fft, nufft
+from ducc_amd import _lib, fft, nufft
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +77,44 @@ def test_long_rows_nufft(n, eps, dtype, coord):
                        fft_order=fo)
         e = E @ c
         assert np.linalg.norm(v.cpu().numpy() - e) <= lim * np.linalg.norm(e)
+
+
+def c2c_factor(a, out, axes, forward, fct):
+    """dmx_c2c with any factor (the Python call has 1, 1/N and 1/sqrt N)"""
+    da, ka = _lib.describe(a)
+    do, ko = _lib.describe(out)
+    ax = np.asarray(axes, dtype=np.int64)
+    opt = _lib.options(stream=torch.cuda.current_stream().cuda_stream)
+    _lib.check(_lib.lib().dmx_c2c(ct.byref(da), ct.byref(do), ax.ctypes.data,
+                                  len(axes), int(forward), float(fct), 1,
+                                  ct.byref(opt)))
+
+
+# (shape, axes): lines in LDS; strided lines; the two column passes; two
+# passes over long lines; global passes; Bluestein first and last; an axis of
+# length 1 alone
+@pytest.mark.parametrize("shape,axes", [
+    ((5, 64), [1]), ((64, 5), [0]), ((1024, 24), [0, 1]), ((2, 16384), [1]),
+    ((20000, 3), [0]), ((3, 1009), [1]), ((12, 101), [0, 1]), ((1, 7), [0])])
+@pytest.mark.parametrize("dtype", [torch.complex64, torch.complex128])
+def test_factor(shape, axes, dtype):
+    """out = fct * DFT(in) for every factor, zero among them, whichever step
+    applies it: contiguous, strided and real input, out of place and in
+    place"""
+    g = torch.Generator(device="cuda").manual_seed(7)
+    n = int(np.prod([shape[a] for a in axes]))
+    a = torch.randn(shape, dtype=dtype, device="cuda", generator=g)
+    wide = torch.zeros((shape[0], 2 * shape[1]), dtype=dtype, device="cuda")
+    wide[:, ::2] = a
+    for x in (a, wide[:, ::2], a.real.contiguous()):
+        e = torch.fft.fftn(x.to(torch.complex128), dim=axes)
+        for fct in (0.0, 0.3, -2.0, 1.0):
+            # (not a zero-filled array: every element has to be written)
+            out = torch.full(shape, 3.0, dtype=dtype, device="cuda")
+            c2c_factor(x, out, axes, True, fct)
+            d = (out - fct * e).norm().item()
+            assert d <= abs(fct) * 4 * tol(dtype, n) * e.norm().item(), fct
+            if x is a:
+                y = x.clone()
+                c2c_factor(y, y, axes, True, fct)
+                assert torch.equal(y, out)
