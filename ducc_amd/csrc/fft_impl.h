@@ -519,7 +519,9 @@ k_fft(FftArgs p) {
 
 }  // namespace
 
-// launches the kernel of one compute type and workgroup size
+// launches the kernel of one compute type and workgroup size (the odd line
+// stride takes full-size workgroups of even lines up to 128 bytes past the
+// default 64 KiB: 16 lines of 512, 8 of 1024, ...)
 template <typename T, int MAXEL>
 void launch_k_fft(const FftArgs &a, int sign, dim3 grid, size_t lds,
                   hipStream_t s);
@@ -529,12 +531,15 @@ void launch_k_fft(const FftArgs &a, int sign, dim3 grid, size_t lds,
   template <>                                                               \
   void launch_k_fft<T, MAXEL>(const FftArgs &a, int sign, dim3 grid,        \
                               size_t lds, hipStream_t s) {                  \
-    if (sign < 0)                                                           \
+    if (sign < 0) {                                                         \
+      allow_big_lds(k_fft<T, MAXEL, -1>, lds);                              \
       hipLaunchKernelGGL((k_fft<T, MAXEL, -1>), grid, dim3(FFT_THREADS),    \
                          lds, s, a);                                        \
-    else                                                                    \
+    } else {                                                                \
+      allow_big_lds(k_fft<T, MAXEL, 1>, lds);                               \
       hipLaunchKernelGGL((k_fft<T, MAXEL, 1>), grid, dim3(FFT_THREADS),     \
                          lds, s, a);                                        \
+    }                                                                       \
     DMX_HIP(hipGetLastError());                                             \
   }                                                                         \
   }

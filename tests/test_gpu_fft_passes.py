@@ -118,3 +118,66 @@ def test_factor(shape, axes, dtype):
                 y = x.clone()
                 c2c_factor(y, y, axes, True, fct)
                 assert torch.equal(y, out)
+
+
+@pytest.mark.parametrize("dtype", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("shape,ax", [
+    ((512, 8203), 0), ((256, 9001), 0), ((630, 517), 0), ((1021, 84), 1),
+    ((4001, 110), 1), ((9, 1 << 18), 1), ((3, 1 << 20), 1)])
+def test_full_workgroups(shape, ax, dtype):
+    """as many lines as a workgroup takes, the last one partly filled:
+    strided and contiguous lines, and both passes of long ones (their
+    padded lines take more than 64 KiB of LDS)"""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a = torch.randn(shape, dtype=dtype, device="cuda", generator=g)
+    r = fft.c2c(a, axes=[ax])
+    e = torch.fft.fft(a.to(torch.complex128), dim=ax)
+    assert ((r - e).norm() / e.norm()).item() < tol(dtype, shape[ax])
+
+
+def kernel_row(W, ofactor, ndim, single):
+    """index of a row of the kernel table"""
+    import csv
+    import os
+    path = os.path.join(os.path.dirname(nufft.__file__), "data",
+                        "kernel_db.csv")
+    rows = [r for r in csv.reader(open(path)) if not r[0].startswith("#")]
+    i = [k for k, r in enumerate(rows)
+         if int(r[0]) == W and float(r[1]) == ofactor and int(r[5]) == ndim
+         and int(r[6]) == int(single)]
+    assert len(i) == 1
+    return i[0]
+
+
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n0,rest", [
+    (255, (100, 120)), (511, (8, 9)), (1023, (8, 9)), (2047, (8, 9))])
+def test_full_workgroups_3d(gpu, n0, rest, dtype):
+    """3-D grids whose strided axis is 512, 1024, 2048 or 4096 long: full
+    workgroups with padded lines, both types"""
+    single = dtype == np.complex64
+    idx = kernel_row(6 if single else 9, 2.0, 3, single)
+    shape = (n0,) + rest
+    rng = np.random.default_rng(n0)
+    M = 2000
+    c = rng.uniform(-np.pi, np.pi, (M, 3))
+    p = (rng.standard_normal(M) + 1j * rng.standard_normal(M)).astype(dtype)
+    q = (rng.standard_normal(shape) +
+         1j * rng.standard_normal(shape)).astype(dtype)
+    out = np.empty(shape, dtype)
+    info = {}
+    nufft.nu2u(points=p, coord=c, forward=True, epsilon=1e-3, out=out,
+               kernel_idx=idx, info=info)
+    assert info["nover"][0] == 2 * (n0 + 1)
+    # the row's error (2e-5 and 3e-8 of the result's norm) over 64 entries
+    lim = 2 * info["eps_tab"] + (2e-6 if single else 0)
+    sel = rng.integers(0, out.size, 64)
+    ref = nufft.nudft_direct(1, c, p, shape, True, sel)
+    rms = np.linalg.norm(out) / np.sqrt(out.size)
+    assert np.linalg.norm(out.reshape(-1)[sel] - ref) <= lim * 8 * rms
+    v = nufft.u2nu(grid=q, coord=c, forward=False, epsilon=1e-3,
+                   kernel_idx=idx)
+    sel = np.arange(64)
+    ref = nufft.nudft_direct(2, c, q, shape, False, sel)
+    rms = np.linalg.norm(v) / np.sqrt(M)
+    assert np.linalg.norm(v[sel] - ref) <= lim * 8 * rms
