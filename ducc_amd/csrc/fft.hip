@@ -299,14 +299,14 @@ int fft_split_long(int L, bool fp64) {
 // (element n1 * L2 + n2): A transforms the columns, neighbouring n2 side by
 // side, B the rows, whose results k1 + L1 * k2 lie side by side for
 // neighbouring k1; both passes read and write runs of neighbours.  The
-// general alternative is one trip through memory per radix.
+// general alternative is one trip through memory per radix.  A launch's
+// second and third index hold 65535 lines each: a larger set takes several
+// pairs of launches.
 bool fft_long_2pass(const FftLaunch &p, int L1, void *dst, bool fp64,
                     const void *tw_L1, const void *tw_L2, const void *tw_L,
                     hipStream_t s, void *a_dst) {
   const int L = p.L, L2 = L / L1;
-  if (L1 < 2 || L1 * L2 != L || p.st_ax != 1 || p.nu > 65535 ||
-      p.nv > 65535)
-    return false;
+  if (L1 < 2 || L1 * L2 != L || p.st_ax != 1) return false;
   const int maxel = fp64 ? FFT_MAXEL64 : FFT_MAXEL32, seg = fp64 ? 8 : 16;
   auto lines = [&](int Ls, int n) {
     int Bl = std::min(maxel / Ls, std::max(seg, maxel / 2 / Ls));
@@ -315,43 +315,50 @@ bool fft_long_2pass(const FftLaunch &p, int L1, void *dst, bool fp64,
     return std::max(1, std::min(Bl, n));
   };
   void *amid = a_dst ? a_dst : p.data;
-  FftArgs c{};
-  c.un1 = p.un1; c.ua1 = p.ua1; c.ua2 = p.ua2;
-  c.on1 = p.vn1; c.oa1 = p.va1; c.oa2 = p.va2;
-  c.st_o = p.st_v;
-  c.in_u = c.out_u = p.st_u;
-  c.tw_full = tw_L;
-  c.bf_in = c.bf_mid = c.bf_out = 1;
-  c.src = p.src ? p.src : p.data;
-  c.scale = p.scale;
-  c.dst = amid;
-  c.Ls = L1;
-  c.tw = tw_L1;
-  c.twiddle = 2;
-  c.nv = c.vn1 = L2;
-  c.Bl = lines(L1, L2);
-  c.in_b = c.out_b = 1;
-  c.in_e = c.out_k = L2;
-  c.kn1 = p.kn1; c.kspan = p.kprune ? p.ka2 - p.kn1 : 0;
-  c.nin_b = 1; c.nin_e = L2;
-  launch_fft(c, fp64, p.sign, (unsigned)p.nu, (unsigned)p.nv, s);
-  c.src = amid;
-  c.scale = 1.0;
-  c.dst = dst;
-  c.Ls = L2;
-  c.tw = tw_L2;
-  c.twiddle = 0;
-  c.nv = c.vn1 = L1;
-  c.Bl = lines(L2, L1);
-  c.in_b = L2;
-  c.in_e = 1;
-  c.out_b = 1;
-  c.out_k = L1;
-  c.kspan = 0;
-  c.nout_b = 1; c.nout_k = L1;
-  c.sn1 = p.sn1; c.sspan = p.sprune ? p.sa2 - p.sn1 : 0;
-  c.bf_in = 0;
-  launch_fft(c, fp64, p.sign, (unsigned)p.nu, (unsigned)p.nv, s);
+  constexpr int MOST = 65535;
+  // lines (u0 + i, v0 + j) of the set, i < nu, j < nv
+  auto part = [&](int u0, int nu, int v0, int nv) {
+    FftArgs c{};
+    c.un1 = p.un1 - u0; c.ua1 = p.ua1 + u0; c.ua2 = p.ua2;
+    c.on1 = p.vn1 - v0; c.oa1 = p.va1 + v0; c.oa2 = p.va2;
+    c.st_o = p.st_v;
+    c.in_u = c.out_u = p.st_u;
+    c.tw_full = tw_L;
+    c.bf_in = c.bf_mid = c.bf_out = 1;
+    c.src = p.src ? p.src : p.data;
+    c.scale = p.scale;
+    c.dst = amid;
+    c.Ls = L1;
+    c.tw = tw_L1;
+    c.twiddle = 2;
+    c.nv = c.vn1 = L2;
+    c.Bl = lines(L1, L2);
+    c.in_b = c.out_b = 1;
+    c.in_e = c.out_k = L2;
+    c.kn1 = p.kn1; c.kspan = p.kprune ? p.ka2 - p.kn1 : 0;
+    c.nin_b = 1; c.nin_e = L2;
+    launch_fft(c, fp64, p.sign, (unsigned)nu, (unsigned)nv, s);
+    c.src = amid;
+    c.scale = 1.0;
+    c.dst = dst;
+    c.Ls = L2;
+    c.tw = tw_L2;
+    c.twiddle = 0;
+    c.nv = c.vn1 = L1;
+    c.Bl = lines(L2, L1);
+    c.in_b = L2;
+    c.in_e = 1;
+    c.out_b = 1;
+    c.out_k = L1;
+    c.kspan = 0;
+    c.nout_b = 1; c.nout_k = L1;
+    c.sn1 = p.sn1; c.sspan = p.sprune ? p.sa2 - p.sn1 : 0;
+    c.bf_in = 0;
+    launch_fft(c, fp64, p.sign, (unsigned)nu, (unsigned)nv, s);
+  };
+  for (int u0 = 0; u0 < p.nu; u0 += MOST)
+    for (int v0 = 0; v0 < p.nv; v0 += MOST)
+      part(u0, std::min(MOST, p.nu - u0), v0, std::min(MOST, p.nv - v0));
   return true;
 }
 

@@ -1055,12 +1055,12 @@ bool Plan::run_fft(bool forward, bool type1, const GridCopyArgs *crop) {
     if (route == FftRoute::rows) {
       void *other = cur_ == grid_.p ? scratch_.p : grid_.p;
       const int L1 = fft_split_long(L.L, p_.fp64);
-      if (fft_long_2pass(L, L1, other, p_.fp64, twiddle_for(L1),
-                         twiddle_for(L.L / L1), twiddle_for(L.L), s_)) {
-        cur_ = other;
-        continue;
-      }
-      DMX_ASSERT(false, "FFT line set too large");
+      const bool ran =
+          fft_long_2pass(L, L1, other, p_.fp64, twiddle_for(L1),
+                         twiddle_for(L.L / L1), twiddle_for(L.L), s_);
+      DMX_ASSERT(ran, "internal: two-pass FFT over rows");
+      cur_ = other;
+      continue;
     }
     L.tw = twiddle_for(L.L);
     fft_lineset(L, p_.fp64, cur_ == grid_.p ? scratch_.p : grid_.p, s_);

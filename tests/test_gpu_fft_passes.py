@@ -181,3 +181,43 @@ def test_full_workgroups_3d(gpu, n0, rest, dtype):
     ref = nufft.nudft_direct(2, c, q, shape, False, sel)
     rms = np.linalg.norm(v) / np.sqrt(M)
     assert np.linalg.norm(v[sel] - ref) <= lim * 8 * rms
+
+
+def test_many_long_lines(gpu):
+    """more than 65535 lines beyond LDS (4096 elements in double precision),
+    by themselves and as the rows of a 2-D grid"""
+    n, L = 65536 + 70, 4116
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = torch.randn((n, L), dtype=torch.complex128, device="cuda",
+                    generator=g)
+    rows = [0, 1, 65534, 65535, 65536, n - 1]
+    e = torch.fft.fft(a[rows], dim=1)
+    r = fft.c2c(a, axes=[1], out=a)
+    for i, q in enumerate(rows):
+        d = ((r[q] - e[i]).norm() / e[i].norm()).item()
+        assert d < tol(torch.complex128, L), q
+    del a, r
+    shape = (33000, 2048)
+    idx = kernel_row(5, 2.0, 2, False)
+    rng = np.random.default_rng(1)
+    M = 50
+    c = torch.from_numpy(rng.uniform(-np.pi, np.pi, (M, 2))).cuda()
+    E = [torch.polar(torch.ones((), dtype=torch.float64, device="cuda"),
+                     torch.outer(c[:, d], torch.arange(
+                         s, dtype=torch.float64, device="cuda") - s // 2))
+         for d, s in enumerate(shape)]
+    p = torch.randn(M, dtype=torch.complex128, device="cuda", generator=g)
+    info = {}
+    out = torch.empty(shape, dtype=torch.complex128, device="cuda")
+    nufft.nu2u(points=p, coord=c, forward=False, epsilon=1e-3, out=out,
+               kernel_idx=idx, info=info)
+    assert info["nover"][0] > 65535 and info["nover"][1] == L
+    lim = 2 * info["eps_tab"]
+    ref = (E[0] * p[:, None]).T.contiguous() @ E[1]
+    assert (out - ref).norm().item() <= lim * ref.norm().item()
+    q = torch.randn(shape, dtype=torch.complex128, device="cuda",
+                    generator=g)
+    v = nufft.u2nu(grid=q, coord=c, forward=False, epsilon=1e-3,
+                   kernel_idx=idx)
+    ref = ((E[0] @ q) * E[1]).sum(1)
+    assert (v - ref).norm().item() <= lim * ref.norm().item()
