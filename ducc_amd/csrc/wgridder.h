@@ -40,7 +40,8 @@ struct WgPoints {
 
 // w planes: w_p = wmin + p dw, kernel support W, FP64 coefficients; the
 // visibilities are sorted by (tile, first plane / step), nk = nplanes / step
-// keys a tile (step > 1 only where tiles * planes exceed 2^30)
+// (rounded up) keys a tile (step > 1 only where tiles * planes exceed 2^24
+// and twice the visibilities)
 struct WgPlanes {
   double wmin, dw;
   int nplanes, W, nk, step;

@@ -583,9 +583,16 @@ void WgJob::choose(double eps, double smin, double smax, bool fp64_values,
 void WgJob::sort_planes(Plan &pln) {
   // stable sort by (tile, first plane), the start of every key
   const size_t nt = pln.ntiles();
+  // (tile, plane) keys: at most 2^24 (a table of 64 MiB) or two a
+  // visibility, and within the sort's 32 bits.  Beyond that (few
+  // visibilities on a large image with thousands of planes) neighbouring
+  // planes share a key, and a plane's subproblems bring visibilities that
+  // have no weight there.
   pl.step = 1;
   auto nk = [&] { return (pl.nplanes + pl.step - 1) / pl.step; };
-  while (nt * (size_t)nk() > ((size_t)1 << 30)) pl.step *= 2;
+  const size_t most =
+      std::min(std::max((size_t)1 << 24, 2 * M), (size_t)1 << 30);
+  while (nt * (size_t)nk() > most && pl.step < pl.nplanes) pl.step *= 2;
   pl.nk = nk();
   const size_t ntab = nt * (size_t)pl.nk + 1;
   idx_.stream = s;

@@ -173,6 +173,96 @@ def test_torch_arrays_and_all_masked(gpu):
     assert np.all(v0 == 0)
 
 
+def _both(uvw, vis, wgt, mask, dirty, px, eps, lim, **kw):
+    """vis2dirty and dirty2vis (frequency c: uvw in wavelengths) against the
+    direct sums"""
+    from ducc_amd import wgridder as W
+    nx, ny = dirty.shape
+    freq = np.array([C])
+    d = W.vis2dirty(uvw=uvw, freq=freq, vis=vis, wgt=wgt, npix_x=nx,
+                    npix_y=ny, pixsize_x=px, pixsize_y=px, epsilon=eps,
+                    do_wgridding=True, mask=mask, **kw)
+    r = G.vis2dirty(uvw, freq, vis, wgt, nx, ny, px, px, True, mask)
+    assert O.l2error(d.astype(complex), r.astype(complex)) <= lim
+    v = W.dirty2vis(uvw=uvw, freq=freq, dirty=dirty, wgt=wgt, pixsize_x=px,
+                    pixsize_y=px, epsilon=eps, do_wgridding=True, mask=mask,
+                    **kw)
+    r = G.dirty2vis(uvw, freq, dirty, wgt, px, px, True, mask)
+    assert O.l2error(v.astype(np.complex128), r) <= lim
+    assert np.all(v[mask == 0] == 0)
+
+
+@pytest.mark.parametrize("single,eps", [(False, 1e-9), (False, 1e-4),
+                                        (True, 1e-4)])
+def test_plane_order(gpu, single, eps):
+    """visibilities by (tile, first plane): a tile with more of a plane's
+    visibilities than one subproblem holds, over a hundred planes (several
+    batches of lists), a gap of planes without any, masked ones"""
+    rng = np.random.default_rng(11)
+    nx, ny, n = 100, 60, 4000
+    px = np.radians(10.) / nx  # dw is about 100 wavelengths
+    uvw = (rng.random((n, 3)) - 0.5) / px
+    w = np.where(rng.random(n) < 0.5, rng.uniform(-2000, 0, n),
+                 rng.uniform(6000, 9000, n))
+    uvw[:, 2] = w
+    uvw[:2500] = [0.1 / px, -0.2 / px, 7000.] + rng.random((2500, 3)) * [
+        0.01 / px, 0.01 / px, 200.]
+    vis = rng.random((n, 1)) - 0.5 + 1j * (rng.random((n, 1)) - 0.5)
+    wgt = rng.uniform(0.9, 1.1, (n, 1))
+    mask = (rng.random((n, 1)) > 0.2).astype(np.uint8)
+    dirty = rng.random((nx, ny)) - 0.5
+    if single:
+        vis, wgt, dirty = (vis.astype(np.complex64), wgt.astype(np.float32),
+                           dirty.astype(np.float32))
+    _both(uvw, vis, wgt, mask, dirty, px, eps, eps)
+
+
+def test_planes_sharing_a_key(gpu):
+    """few visibilities, many tiles and planes: more than 2^24 (tile, plane)
+    pairs, so that neighbouring planes share a sort key (and more planes than
+    are counted in LDS)"""
+    rng = np.random.default_rng(12)
+    nx, n, eps, sigma = 320, 40, 1e-6, 2.0
+    px = np.radians(20.) / nx
+    uvw = (rng.random((n, 3)) - 0.5) / px
+    # n - 1 runs from 0 to that of the corner, centred by the shift
+    nm1 = 1 - np.sqrt(1 - 2 * (nx / 2 * px) ** 2)
+    dw = 0.5 / sigma / (0.5 * nm1)
+    # clusters over 60000 planes, some a fraction of a plane wide
+    uvw[:, 2] = np.repeat(rng.uniform(-3e4, 3e4, 8), 5) * dw + \
+        rng.uniform(0, 1, n) * np.repeat([0.1, 1, 2, 3, 4, 9, 20, 40], 5) * dw
+    uvw[0, 2], uvw[1, 2] = -3e4 * dw, 3e4 * dw
+    tiles = (2 * nx // 32) ** 2  # 32 x 32 cells each
+    assert tiles * 6e4 > 1 << 24
+    vis = rng.random((n, 1)) - 0.5 + 1j * (rng.random((n, 1)) - 0.5)
+    mask = np.ones((n, 1), np.uint8)
+    mask[7] = 0
+    dirty = rng.random((nx, nx)) - 0.5
+    # rounding of phases of w (n - 1) turns: 2 pi 4e3 * 1.1e-16
+    _both(uvw, vis, np.ones((n, 1)), mask, dirty, px, eps, eps + 1e-11,
+          sigma_min=sigma, sigma_max=sigma)
+
+
+def test_key_table_is_bounded(gpu):
+    """device memory of a call goes with its image and visibilities, not
+    with tiles times planes (1.8 GB of table here at one entry each)"""
+    from ducc_amd import wgridder as W
+    nx, n, sigma = 1400, 16, 2.0
+    px = np.radians(20.) / nx
+    nm1 = 1 - np.sqrt(1 - 2 * (nx / 2 * px) ** 2)
+    dw = 0.5 / sigma / (0.5 * nm1)
+    uvw = np.zeros((n, 3))
+    uvw[: n // 2, 2], uvw[n // 2:, 2] = -3e4 * dw, 3e4 * dw
+    assert (2 * nx // 32) ** 2 * 6e4 * 4 > 1.7e9
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    W.vis2dirty(uvw=uvw, freq=np.array([C]), vis=np.ones((n, 1), complex),
+                npix_x=nx, npix_y=nx, pixsize_x=px, pixsize_y=px,
+                epsilon=1e-6, do_wgridding=True, sigma_min=sigma,
+                sigma_max=sigma)
+    assert free - torch.cuda.mem_get_info()[0] < 1 << 30
+
+
 def test_errors(gpu):
     from ducc_amd import wgridder as W
     px, py, freq, uvw, ms, wgt, mask, dirty = _problem(1, 8, 8, 4, 2, 1.0)
