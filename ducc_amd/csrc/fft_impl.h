@@ -69,32 +69,72 @@ template <> struct Tw<11> {
       -0.54064081745559758211};
 };
 
-// exp(2 pi i k / R) for the composite radices with inner twiddles
-template <> struct Tw<9> {
-  static constexpr double c[5] = {1.0, 0.76604444311897803520,
-                                  0.17364817766693034885, -0.5,
-                                  -0.93969262078590838405};
-  static constexpr double s[5] = {0.0, 0.64278760968653932632,
-                                  0.98480775301220805936,
-                                  0.86602540378443864676,
-                                  0.34202014332566873304};
-};
-template <> struct Tw<16> {
-  static constexpr double c[10] = {1.0, 0.92387953251128675613,
-                                   0.70710678118654752440,
-                                   0.38268343236508977173, 0.0,
-                                   -0.38268343236508977173,
-                                   -0.70710678118654752440,
-                                   -0.92387953251128675613, -1.0,
-                                   -0.92387953251128675613};
-  static constexpr double s[10] = {0.0, 0.38268343236508977173,
-                                   0.70710678118654752440,
-                                   0.92387953251128675613, 1.0,
-                                   0.92387953251128675613,
-                                   0.70710678118654752440,
-                                   0.38268343236508977173, 0.0,
-                                   -0.38268343236508977173};
-};
+// a turned by an angle of tan(angle / 2) = t and sin(angle) = s: three
+// shears, each a fused multiply-add that rounds once
+template <typename T, typename C>
+__device__ __forceinline__ C shear3(C a, T t, T s) {
+  a.x -= t * a.y;
+  a.y += s * a.x;
+  a.x -= t * a.y;
+  return a;
+}
+
+// a * exp(sign 2 pi i m / R), the inner twiddles of R = 9 and 16: a small
+// turn by shears, then quarter turns; 45 degrees as in radix 8.  Full complex
+// products rounded twice as often and, in single precision, took a cosine of
+// 22.5 degrees that is off by half a unit: rows of 4096 came out at 1.22e-7
+// (1.19e-7 with radix 8 and a pass more), with the turns at 1.15e-7; rows of
+// 729 at 1.30e-7 (1.29e-7 with radix 3), with the turns at 1.25e-7.  Times
+// of 2-D and 3-D calls are the same; a 1-D call of two latency-bound passes
+// (u2nu, 100003 modes) went 80.6 -> 81.4 us.
+template <typename T, int R, typename C>
+__device__ __forceinline__ C turn(C a, int m, int sign) {
+  const T sg = (T)sign;
+  if constexpr (R == 16) {
+    const T h = (T)0.70710678118654752440;
+    const T t = sg * (T)0.19891236737965800691,  // tan(pi/16)
+        s = sg * (T)0.38268343236508977173;      // sin(pi/8)
+    C r;
+    switch (m) {
+      case 1: return shear3<T>(a, t, s);
+      case 2:
+        r.x = (a.x - sg * a.y) * h;
+        r.y = (a.y + sg * a.x) * h;
+        return r;
+      case 3: return cmuli(shear3<T>(a, -t, -s), sign);
+      case 4: return cmuli(a, sign);
+      case 6:
+        r.x = (-a.x - sg * a.y) * h;
+        r.y = (-a.y + sg * a.x) * h;
+        return r;
+      case 9:
+        r = shear3<T>(a, t, s);
+        r.x = -r.x;
+        r.y = -r.y;
+        return r;
+      default: return a;  // 0
+    }
+  } else {
+    static_assert(R == 9, "turns of 40 degrees");
+    C r;
+    switch (m) {
+      case 1:  // 40 degrees: tan 20, sin 40
+        return shear3<T>(a, sg * (T)0.36397023426620236135,
+                         sg * (T)0.64278760968653932632);
+      case 2:  // 90 - 10
+        return cmuli(shear3<T>(a, -sg * (T)0.08748866352592400522,
+                               -sg * (T)0.17364817766693034885),
+                     sign);
+      case 4:  // 180 - 20
+        r = shear3<T>(a, -sg * (T)0.17632698070846497347,
+                      -sg * (T)0.34202014332566873304);
+        r.x = -r.x;
+        r.y = -r.y;
+        return r;
+      default: return a;  // 0
+    }
+  }
+}
 
 // the two factors of a composite radix (0: none)
 constexpr int radix_a(int R) {
@@ -174,16 +214,8 @@ __device__ __forceinline__ void dft(C *v, int sign) {
       for (int n1 = 0; n1 < A; ++n1) t[n1] = v[A * n1 + n2];
       dft<T, A>(t, sign);
 #pragma unroll
-      for (int k1 = 0; k1 < A; ++k1) {
-        if (n2 * k1 == 0) {
-          y[n2][k1] = t[k1];
-        } else {
-          C w;
-          w.x = (T)Tw<R>::c[n2 * k1];
-          w.y = (T)sign * (T)Tw<R>::s[n2 * k1];
-          y[n2][k1] = cmul(t[k1], w);
-        }
-      }
+      for (int k1 = 0; k1 < A; ++k1)
+        y[n2][k1] = turn<T, R>(t[k1], n2 * k1, sign);
     }
 #pragma unroll
     for (int k1 = 0; k1 < A; ++k1) {

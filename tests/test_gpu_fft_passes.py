@@ -19,9 +19,18 @@ LENGTHS = [2, 3, 5, 6, 7, 9, 10, 11, 12, 14, 15, 16, 84, 110, 210, 432, 462,
 
 
 def tol(dtype, n):
-    """rounding of log2(n) butterfly levels and their twiddles, in rms"""
-    eps = 1.2e-7 if dtype == torch.complex64 else 2.3e-16
-    return 4 * eps * np.log2(max(n, 2))
+    """Relative error in rms of log2(n) butterfly levels that each round once
+    or twice by up to u, half a unit, independently: about u sqrt(log2 n).
+    Measured over all lengths here: 0.5 to 0.92 of that in single precision,
+    0.5 to 1.5 in double, where the comparison's own error adds.  Bluestein
+    (a prime factor above 11): three transforms of twice the length."""
+    u = 6e-8 if dtype == torch.complex64 else 1.11e-16
+    t = u * np.sqrt(max(np.log2(n), 1.0))
+    for p in (2, 3, 5, 7, 11):
+        while n % p == 0:
+            n //= p
+    return t * (1.3 if dtype == torch.complex64 else 2.0) * (
+        1.0 if n == 1 else 2.0)
 
 
 @pytest.mark.parametrize("dtype", [torch.complex64, torch.complex128])
@@ -39,8 +48,7 @@ def test_lines(n, dtype):
             f = torch.fft.fft if fwd else torch.fft.ifft
             e = f(a.to(torch.complex128), dim=ax)
             err = ((r - e).norm() / e.norm()).item()
-            # Bluestein: three transforms of twice the length
-            assert err < tol(dtype, n) * (4 if n == 16381 else 1), (shape, err)
+            assert err < tol(dtype, n), (shape, err)
             assert torch.equal(a, keep)
 
 
@@ -113,7 +121,8 @@ def test_factor(shape, axes, dtype):
             out = torch.full(shape, 3.0, dtype=dtype, device="cuda")
             c2c_factor(x, out, axes, True, fct)
             d = (out - fct * e).norm().item()
-            assert d <= abs(fct) * 4 * tol(dtype, n) * e.norm().item(), fct
+            # (the factor rounds once more)
+            assert d <= abs(fct) * 2 * tol(dtype, n) * e.norm().item(), fct
             if x is a:
                 y = x.clone()
                 c2c_factor(y, y, axes, True, fct)
@@ -221,3 +230,21 @@ def test_many_long_lines(gpu):
                    kernel_idx=idx)
     ref = ((E[0] @ q) * E[1]).sum(1)
     assert (v - ref).norm().item() <= lim * ref.norm().item()
+
+
+@pytest.mark.parametrize("shape,ax,most", [
+    ((512, 4096), 1, 1.19e-7), ((2048, 2048), 1, 1.124e-7),
+    ((81, 4096), 0, 1.01e-7), ((4096, 729), 1, 1.285e-7)])
+def test_wide_radices_round_no_more(shape, ax, most):
+    """single precision: lines of radices 16 and 9 are no further from the
+    64-bit transform than with radices 8 and 3 (`most`)"""
+    s = q = 0.0
+    for seed in range(3):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        a = torch.randn(shape, dtype=torch.complex64, device="cuda",
+                        generator=g)
+        r = fft.c2c(a, axes=[ax])
+        e = torch.fft.fft(a.to(torch.complex128), dim=ax)
+        s += (r - e).norm().item() ** 2
+        q += e.norm().item() ** 2
+    assert np.sqrt(s / q) <= most
