@@ -7,27 +7,55 @@ namespace dmx {
 namespace {
 constexpr unsigned INTERP_MAX_BLOCKS = 8192;
 
+// 3-D: 512 threads instead of 256 share a region.
+// * 16^3 tiles (on request): always, once the region exceeds a third of the
+//   LDS (W = 4, 6 in FP32: 3-4 % and 11-19 % faster; W = 5 in FP64: 15-27 %).
+// * 8^3 tiles: only where one region alone fits a CU, which then has eight
+//   waves instead of four: FP64 gradients with W = 10 to 13.  96x100x108
+//   modes, 256 -> 512 threads: W = 11 and 12 gain at any density (1e6
+//   clustered points 2.69 -> 2.11 ms, 1e6 uniform 5.41 -> 5.12, 6e6 uniform
+//   10.3 -> 7.2); W = 10 and 13 gain at 250 points a tile (6.62 -> 5.57 and
+//   16.0 -> 12.1 ms) and lose at 40 (3.59 -> 3.96 and 8.31 -> 8.60).  Where
+//   two regions fit, one workgroup of 512 threads takes the registers of
+//   two: W = 8 values 0.57 -> 0.65 ms, gradients of W = 8 and 9 1.50 -> 2.37
+//   and 1.83 -> 3.07 ms.
+// * 4^3 tiles (W >= 14) have too few points for them (5 % slower).
+bool wide_workgroup(const SpreadArgs &a, size_t sh) {
+  if (a.g.ndim != 3 || sh <= LDS_MAX_BYTES / 3) return false;
+  if (a.g.log2tile != 3) return a.g.log2tile > 3;
+  if (sh <= LDS_MAX_BYTES / 2 || a.g.W < 10) return false;
+  if (a.g.W == 11 || a.g.W == 12) return true;
+  // a hundred points a tile: subproblems beyond one per tile
+  const size_t nt = (size_t)a.g.ntiles[0] * a.g.ntiles[1] * a.g.ntiles[2];
+  return a.nsub_max > nt + nt * 100 / MAXSUB;
+}
+
 template <typename T, int NDIM, int W, int MODE>
 void go(const SpreadArgs &a, void *out, int out_f64, hipStream_t s) {
   unsigned nb = (unsigned)std::min<size_t>(a.nsub_max, INTERP_MAX_BLOCKS);
   if (nb == 0) return;
+  // 3-D FP64 values with W >= 9 in LDS are launch_interp_wave's
+  constexpr bool wave = NDIM == 3 && sizeof(T) == 8 && MODE == 0 && W >= 9;
   if (a.use_lds) {
-    size_t cells = interp_inner_pad(a.lds_side);
-    for (int d = 1; d < NDIM; ++d) cells *= a.lds_side;
-    size_t sh = 2 * cells * sizeof(T);
-    // a region of more than a third of the CU's LDS: 512 threads share it
-    if constexpr (NDIM == 3) {
-      if (sh > LDS_MAX_BYTES / 3) {
-        allow_big_lds(k_interp<T, NDIM, W, true, MODE, 512>, sh);
-        hipLaunchKernelGGL((k_interp<T, NDIM, W, true, MODE, 512>), dim3(nb),
-                           dim3(512), sh, s, a, out, out_f64);
-        DMX_HIP(hipGetLastError());
-        return;
+    if constexpr (wave) {
+      throw Error("internal: region of a wide kernel beyond LDS");
+    } else {
+      size_t cells = interp_inner_pad(a.lds_side);
+      for (int d = 1; d < NDIM; ++d) cells *= a.lds_side;
+      size_t sh = 2 * cells * sizeof(T);
+      if constexpr (NDIM == 3) {
+        if (wide_workgroup(a, sh)) {
+          allow_big_lds(k_interp<T, NDIM, W, true, MODE, 512>, sh);
+          hipLaunchKernelGGL((k_interp<T, NDIM, W, true, MODE, 512>),
+                             dim3(nb), dim3(512), sh, s, a, out, out_f64);
+          DMX_HIP(hipGetLastError());
+          return;
+        }
       }
+      allow_big_lds(k_interp<T, NDIM, W, true, MODE>, sh);
+      hipLaunchKernelGGL((k_interp<T, NDIM, W, true, MODE>), dim3(nb),
+                         dim3(256), sh, s, a, out, out_f64);
     }
-    allow_big_lds(k_interp<T, NDIM, W, true, MODE>, sh);
-    hipLaunchKernelGGL((k_interp<T, NDIM, W, true, MODE>), dim3(nb), dim3(256),
-                       sh, s, a, out, out_f64);
   } else {
     if constexpr (NDIM == 3)
       hipLaunchKernelGGL((k_interp<T, NDIM, W, false, MODE>), dim3(nb),

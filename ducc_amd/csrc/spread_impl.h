@@ -792,10 +792,7 @@ __host__ __device__ inline int interp_inner_pad(int S) { return (S + 3) & ~1; }
 // The region is staged in LDS as interleaved complex cells (one 8/16-byte
 // read per tap); 2-D FP32 reads aligned pairs of cells (16 bytes) and picks
 // the taps by the parity of the first column.
-// NT: threads per workgroup.  A region above a third of a CU's LDS leaves
-// room for one or two workgroups: they take 512 threads, so that two waves a
-// SIMD are in flight (3-D FP64, W = 11, 104 KB regions, 1e6 clustered
-// points, before those requests went to k_interp_wave: 1400 -> 1050 us).
+// NT: threads per workgroup (256 or 512, chosen and measured in interp.hip).
 template <typename T, int NDIM, int W, bool LDS, int MODE, int NT = 256>
 __global__ __launch_bounds__(NT) void k_interp(SpreadArgs a, void *out,
                                                int out_f64) {

@@ -20,3 +20,14 @@ def gpu():
     from ducc_amd import _lib
     _lib.require_gpu()
     return True
+
+
+def kernel_rows(ofactor, ndim, single):
+    """{W: (index, epsilon)} of the kernel table's rows of an oversampling
+    factor"""
+    import csv
+    path = os.path.join(ROOT, "ducc_amd", "data", "kernel_db.csv")
+    rows = [r for r in csv.reader(open(path)) if not r[0].startswith("#")]
+    return {int(r[0]): (i, float(r[2])) for i, r in enumerate(rows)
+            if float(r[1]) == ofactor and int(r[5]) == ndim
+            and int(r[6]) == int(single)}

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 import torch
 
+from conftest import kernel_rows
 from ducc_amd import _lib, fft, nufft
 
 pytestmark = pytest.mark.gpu
@@ -144,20 +145,6 @@ def test_full_workgroups(shape, ax, dtype):
     assert ((r - e).norm() / e.norm()).item() < tol(dtype, shape[ax])
 
 
-def kernel_row(W, ofactor, ndim, single):
-    """index of a row of the kernel table"""
-    import csv
-    import os
-    path = os.path.join(os.path.dirname(nufft.__file__), "data",
-                        "kernel_db.csv")
-    rows = [r for r in csv.reader(open(path)) if not r[0].startswith("#")]
-    i = [k for k, r in enumerate(rows)
-         if int(r[0]) == W and float(r[1]) == ofactor and int(r[5]) == ndim
-         and int(r[6]) == int(single)]
-    assert len(i) == 1
-    return i[0]
-
-
 @pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
 @pytest.mark.parametrize("n0,rest", [
     (255, (100, 120)), (511, (8, 9)), (1023, (8, 9)), (2047, (8, 9))])
@@ -165,7 +152,7 @@ def test_full_workgroups_3d(gpu, n0, rest, dtype):
     """3-D grids whose strided axis is 512, 1024, 2048 or 4096 long: full
     workgroups with padded lines, both types"""
     single = dtype == np.complex64
-    idx = kernel_row(6 if single else 9, 2.0, 3, single)
+    idx = kernel_rows(2.0, 3, single)[6 if single else 9][0]
     shape = (n0,) + rest
     rng = np.random.default_rng(n0)
     M = 2000
@@ -207,7 +194,7 @@ def test_many_long_lines(gpu):
         assert d < tol(torch.complex128, L), q
     del a, r
     shape = (33000, 2048)
-    idx = kernel_row(5, 2.0, 2, False)
+    idx = kernel_rows(2.0, 2, False)[5][0]
     rng = np.random.default_rng(1)
     M = 50
     c = torch.from_numpy(rng.uniform(-np.pi, np.pi, (M, 2))).cuda()
