@@ -62,6 +62,12 @@ __global__ __launch_bounds__(WT) void k_interp_wave(SpreadArgs a, void *out,
                                                     int chunk) {
   constexpr int NS = (W * W + 63) / 64;  // lane sets of the W x W plane
   constexpr int DP = W + 3 + (W & 1), NE = (DP + 1) / 2, NH = (W + 1) / 2;
+  // Lanes past the plane read its last tap and drop the sum: a branch around
+  // each of their reads, unrolled W times, spilled 40 to 142 registers a lane
+  // at W = 12 to 15.  At W = 14 and 15 that leaves 12 to 15, and the walk with
+  // the branch in a loop that is not unrolled is as fast or faster.
+  constexpr bool MASK = W == 14 || W == 15;
+  constexpr int UN = MASK ? 1 : W;
   extern __shared__ unsigned char smem_raw[];
   const int S = a.lds_side, tile = 1 << a.g.log2tile;
   const int ncell = S * S * SP, plane = S * SP;
@@ -165,12 +171,12 @@ __global__ __launch_bounds__(WT) void k_interp_wave(SpreadArgs a, void *out,
 #pragma unroll
         for (int s = 0; s < NS; ++s) re[s] = im[s] = 0.0;
         const double2 *b = buf + base;
-#pragma unroll
+#pragma unroll UN
         for (int c = 0; c < W; ++c) {
           const double w0 = lane_value(w, c);
 #pragma unroll
           for (int s = 0; s < NS; ++s) {
-            if (s < NS - 1 || last_in) {
+            if (!MASK || s < NS - 1 || last_in) {
               const double2 g = b[c * plane + off[s]];
               re[s] += w0 * g.x;
               im[s] += w0 * g.y;
