@@ -84,8 +84,11 @@ __global__ __launch_bounds__(256) void k_fft_global_pass(FftLaunch p,
 namespace {
 // Radices of the passes of a line of length L: the fewest passes (each is a
 // sweep over LDS and two barriers), then the smallest radices.  allow: bit
-// R set for each usable radix.  Odd radices come first: the first pass
-// writes its results R elements apart, free of bank conflicts for odd R.
+// R set for each usable radix.  In LDS odd radices come first: the first pass
+// writes its results R elements apart, free of bank conflicts for odd R.  In
+// global memory the even ones do, so that the early passes write whole
+// aligned segments (2000376 = 8 7^3 3^6 in FP64: the call's ten passes 284 ->
+// 261 us).
 constexpr uint32_t GLOBAL_RADICES =
     1u << 11 | 1u << 8 | 1u << 7 | 1u << 5 | 1u << 4 | 1u << 3 | 1u << 2;
 constexpr int RADICES[14] = {16, 15, 14, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2};
@@ -112,12 +115,14 @@ void search_radices(int L, int from, int n, int sum, uint32_t allow,
   }
 }
 
-int plan_passes(int L, uint32_t allow, FftPass *pass) {
+int plan_passes(int L, uint32_t allow, FftPass *pass, bool lds = true) {
   int cur[FFT_MAXPASS], f[FFT_MAXPASS], n = FFT_MAXPASS + 1, sum = 0;
   search_radices(L, 0, 0, 0, allow, cur, f, n, sum);
   DMX_ASSERT(n <= FFT_MAXPASS, "FFT length is not 2,3,5,7,11-smooth");
-  std::stable_sort(f, f + n, [](int a, int b) {
-    return (a & 1) != (b & 1) ? (a & 1) > (b & 1) : a > b;
+  std::stable_sort(f, f + n, [lds](int a, int b) {
+    const bool oa = a & 1, ob = b & 1;
+    if (oa != ob) return lds ? oa : ob;
+    return lds || !oa ? a > b : a < b;
   });
   int Ns = 1;
   for (int i = 0; i < n; ++i) {
@@ -402,7 +407,7 @@ void fft_lineset(const FftLaunch &base, bool fp64, void *scratch,
     launch_fft(c, fp64, p.sign, (unsigned)p.nu, 1, s);
     return;
   }
-  p.npass = plan_passes(p.L, GLOBAL_RADICES, p.pass);
+  p.npass = plan_passes(p.L, GLOBAL_RADICES, p.pass, false);
   // long lines: global Stockham passes, ping-pong between data and scratch
   DMX_ASSERT(scratch != nullptr, "internal: FFT scratch missing");
   const void *src = p.src ? p.src : p.data;
