@@ -515,11 +515,15 @@ __device__ __forceinline__ void fft_pass_radix(const FftArgs &p,
 
 // MAXEL: the most elements (lines x length) the launch puts in one
 // workgroup; it sizes the register staging of the passes, and the half-size
-// variant leaves room for more workgroups per CU
+// variant leaves room for more workgroups per CU.  Waves a SIMD: the full-size
+// variants hold twice the staging and two or three of their workgroups fit a
+// CU, so they get the registers of three waves (at 5 and 4 waves, as the
+// half-size ones, they spilled 500 registers a lane in FP32 and 150 in FP64:
+// c2c of 3000^2 in FP64 232 -> 205 us, rows of a 3024^2 FP64 grid 99 -> 82).
 template <typename T, int MAXEL, int SIGN>
 __global__ __launch_bounds__(FFT_THREADS) __attribute__((
     amdgpu_waves_per_eu(
-    sizeof(T) * MAXEL <= 32768 ? (sizeof(T) == 4 ? 5 : 4) : 1))) void
+    sizeof(T) * MAXEL <= 16384 ? (sizeof(T) == 4 ? 5 : 4) : 3))) void
 k_fft(FftArgs p) {
   using C = typename V2<T>::t;
   extern __shared__ unsigned char smem_raw[];
