@@ -944,12 +944,27 @@ void launch_tile_subs(size_t ntiles, uint32_t *counts, uint32_t *tstart,
   DMX_HIP(hipGetLastError());
 }
 
+// Whether one launch or one counting pass over whole keys builds the index.
+// The pass's table has tiles x blocks entries and each of its blocks clears
+// and scans a counter per tile and wave, while the runs it writes get
+// shorter; the 8-bit passes do not depend on the tiles.  Measured where the
+// two meet (uniform points, whole calls): 7e6 points in 1700 tiles, 1.5e6 in
+// 2800, 6e5 in 3950, which is M * tiles^3 = 3.5e16 throughout (400^2 modes,
+// 784 tiles, still gain at 1e7 points: 593 -> 531 us; 950^2, 3969 tiles, 3e6
+// points would take 279 instead of 225, 7e5 in 1-D, 1e7 points in 2740
+// tiles, 648 instead of 554).
+bool index_one_pass(size_t M, size_t ntiles) {
+  if (ntiles > (size_t)WIDE_TILES) return false;
+  const double t = (double)ntiles;
+  return M <= (size_t)SMALL_M || (double)M * t * t * t <= 3.5e16;
+}
+
 bool launch_index(const Geo &g, const void *coords, size_t M, int keybits,
                   size_t ntiles, uint32_t *idx, uint32_t *keys, void *work,
                   uint32_t *counts, uint32_t *tstart, uint32_t *nsub,
                   uint32_t *sub_start, Sub *subs, uint32_t *nsub_total,
                   hipStream_t s) {
-  if (!M || ntiles > (size_t)WIDE_TILES) return false;
+  if (!M || !index_one_pass(M, ntiles)) return false;
 #define DMX_BYDIM(KERNEL, ...)                              \
   switch (g.ndim) {                                         \
     case 1: KERNEL(1, __VA_ARGS__); break;                  \

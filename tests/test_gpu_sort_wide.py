@@ -8,9 +8,10 @@ from oracle import core as O
 
 pytestmark = pytest.mark.gpu
 
-# 4096 points: one workgroup; 2^19: blocks of 1024 / 4096 points
+# 4096 points: one workgroup; 2^19: blocks of 1024 / 4096 points; 3969 tiles
+# take one pass up to 5.6e5 points
 MS = [1, 63, 64, 1025, 4095, 4096, 4097, 5000, 70001, (1 << 19) - 1,
-      (1 << 19) + 1]
+      (1 << 19) + 1, 600_001]
 # (dimensions, grid, log2 tile, W): 11, 36, 4096 - 64 * 3.., 4096+ tiles
 GRIDS = [((4096,), 9, 7), ((110, 84), 5, 8), ((1950, 1950), 5, 7),
          ((1954, 1954), 5, 7), ((1984, 1984), 5, 7), ((100, 100, 100), 3, 6)]
