@@ -2,11 +2,14 @@
 // kernels of fft.hip: the drop-in for ducc0::c2c (src/ducc0/fft/fft.h:
 // 848-850; Python binding python/fft_pymod.cc:122-172).
 //
-// The input is copied (scaled by fct, real input widened to complex) into a
-// contiguous work array, the output itself when that is contiguous.  Each
-// axis is then transformed in place, the array seen as (outer, L, inner):
-//  * L 2,3,5,7,11-smooth: Stockham passes, in LDS when the line fits,
-//    otherwise out-of-place global passes;
+// The work array is the output itself when that is contiguous.  A contiguous
+// complex input is read by the first axis's transform, which applies fct;
+// any other is first copied into the work array (scaled, real input widened
+// to complex).  The other axes are transformed in place, the array seen as
+// (outer, L, inner):
+//  * L 2,3,5,7,11-smooth: Stockham passes, in LDS when the line fits, in
+//    two such passes when it has a split, otherwise out-of-place global
+//    passes;
 //  * any other L: Bluestein's chirp-z algorithm (X_m = w_m sum_k x_k w_k
 //    conj(w_{m-k}), w_k = exp(-/+ i pi k^2 / L)) as a circular convolution
 //    of smooth length n2 >= 2L-1, done with two FFTs of length n2 on an

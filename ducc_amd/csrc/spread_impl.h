@@ -533,7 +533,12 @@ __global__ __launch_bounds__(NT) void k_spread(SpreadArgs a) {
           // keeps the lanes of a quarter-wave on distinct classes).  The
           // split f with the least rounds * (planes + 1), the one for the
           // point's weights: 5 runs (300 points a tile) take 12 instead of
-          // 14 on four waves.
+          // 14 on four waves.  Against splitting below four runs only:
+          // fixed point, W = 6 and 8, 60 to 210 points a tile 1-2 % of a
+          // call (5e7 points in 8^3 tiles, W = 6: spreading 6.06 -> 5.78
+          // ms); FP64 accumulators of FP32 calls 0 to 1.6 % (W = 8, 5e7
+          // points 34.1 -> 33.6 ms); FP64 W = 6, 9, 11 0 to 1.6 %, W = 13
+          // up to 4 %, W = 10 and 14 1 % slower.
           int fl = 0;  // log2 f
           if constexpr (NDIM == 3) {
             int best = 1 << 30;
@@ -683,9 +688,7 @@ __global__ __launch_bounds__(NT) void k_spread(SpreadArgs a) {
         // [W-1, tile) of its region (its neighbours' regions overlap the
         // rest, and the periodic wrap brings other tiles' points only to the
         // first and last nsafe cells of the grid): plain stores onto the
-        // zeroed grid there, atomics elsewhere.  64 x 64 tiles, W = 7: 69 %
-        // of the cells, 93 -> 84 us per w plane of 3.6e5 points on 3750^2
-        // cells.
+        // zeroed grid there, atomics elsewhere.
         auto mine = [&](int o, int d, int n) {
           return o >= W - 1 && o < tile &&
                  (unsigned)(b0[d] + o - a.g.nsafe) <
@@ -730,8 +733,15 @@ __global__ __launch_bounds__(NT) void k_spread(SpreadArgs a) {
           }
         }
         };
-        // (only where these are most of the region's cells: at less, or in
-        // crowded tiles with several subproblems, the test costs 2-5 %)
+        // Only where these are most of the region's cells: 64 x 64 tiles to
+        // W = 13 (W = 7: 69 % of the cells, 93 -> 84 us per w plane of 3.6e5
+        // points on 3750^2 cells), 32 x 32 tiles to W = 6, all 1-D tiles.
+        // Whole calls, atomics -> stores: 2-D FP32, 2e6 points on 2048^2
+        // modes 10 % faster at W = 4, 5, 6 (710 -> 645 us), 512^2 FP64 8-10
+        // %, crowded tiles (several subproblems, atomics all the same) within
+        // 0.6 %; 1-D, 3e5 to 3e6 points on 1e6 modes 2-6 % faster, crowded
+        // 1-D tiles 0-1 % slower, 2 % at W = 11.  With the test and few own
+        // cells (W = 7 in 32 x 32 tiles) calls were 1-2 % slower.
         if (mostly_own && a.tile_nsub[sb.tile] == 1)
           flush(std::integral_constant<bool, true>{});
         else
