@@ -12,10 +12,13 @@
 // rows of W neighbouring cells, the row stride is W modulo 16 so that
 // consecutive lanes stay on consecutive banks over row ends, each lane
 // evaluates one of the 3 W weights (its polynomial stays in registers), and
-// 1024 threads fit.  W = 11, 96x100x108 modes, 1e6 points: 810 us (row
-// stride 19, W modulo 8: 845 us).  Splitting a subproblem over two or four
-// workgroups, each staging the region, cost more than the shorter tail gave
-// (907 and 1050 us).
+// 1024 threads fit.  W = 11, 96x100x108 modes, 1e6 points: 713 us (810 us
+// with a branch around the last lanes' reads; then also: row stride 19, W
+// modulo 8, 845 us, and a subproblem split over two or four workgroups, each
+// staging the region, 907 and 1050 us).  Against one lane per point, whole
+// calls of uniform points on that grid: W = 9 697 -> 537 us (2e4 points), 2.56
+// -> 2.58 ms (6e6); W = 12 1.68 -> 0.65 and 8.9 -> 4.4 ms; W = 15 3.0 -> 0.8
+// and 18.0 -> 7.3 ms; W = 16 3.6 -> 0.9 and 28.5 -> 10.5 ms.
 #include "spread_impl.h"
 
 namespace dmx {
